@@ -27,8 +27,9 @@ LIB = os.path.join(HERE, "libbitcache_hip.so")
 EXT_SUFFIX = sysconfig.get_config_var("EXT_SUFFIX") or ".so"
 EXT = os.path.join(HERE, "_C" + EXT_SUFFIX)
 
-HIP_SOURCES = ["encode.hip", "attention.hip", "attention_mfma.hip", "adaptive.hip", "convert.hip",
-               "probe.hip", "abi.cpp"]
+# (the longest compiles first: the matrix-core attention kernels, one file per head dim)
+HIP_SOURCES = [f"attn_mfma_d{d}.hip" for d in (256, 224, 192, 160, 128, 96, 64, 32)] + [
+    "attention.hip", "adaptive.hip", "encode.hip", "attention_mfma.hip", "convert.hip", "probe.hip", "abi.cpp"]
 HIP_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

@@ -1157,8 +1157,7 @@ int run_partial(int mode, const void* q, const void* k_bin, const void* k_res, c
         a.group_list = lists + kListHeader / sizeof(int32_t);
         a.group_count = lists;
     }
-    const bool mfma = !valu_forced() && bc::mfma_split_ok(head_dim, a.chunk) &&
-                      (head_dim == 64 || head_dim == 128 || head_dim == 256);
+    const bool mfma = !valu_forced() && bc::mfma_split_ok(head_dim, a.chunk);
     // one wide workgroup per head (wide_plan): no partials, no merge launch
     if (mfma && direct_out != nullptr && app == nullptr &&
         wide_plan(mode, head_dim, p.G, groups, seq_len, bc::device_cu_count())) {
@@ -1394,7 +1393,8 @@ extern "C" int bc_append_attention(const void* q, const void* k_new, const void*
     const SplitPlan p = plan_splits(batch, n_heads, n_kv_heads, seq_len,
                                     plan_per_cu(mode, head_dim, pick_g(group)));
     hipStream_t st = (hipStream_t)stream;
-    if (valu_forced() || pick_g(group) != group || !bc::mfma_split_ok(head_dim, p.chunk)) {
+    if (valu_forced() || pick_g(group) != group || !bc::append_dim(head_dim) ||
+        !bc::mfma_split_ok(head_dim, p.chunk)) {
         const int rc = bc_online_encode_kv(k_new, v_new, k_bin, k_res, v_bin, v_res, batch,
                                            n_kv_heads, head_dim, current_len, max_seq, stream);
         if (rc != BC_OK) return rc;

@@ -1,5 +1,5 @@
 // Shared declarations of the split-KV attention kernels (attention.hip,
-// attention_mfma.hip).
+// attn_mfma_kernel.h).
 #pragma once
 
 #include "common.h"
@@ -63,11 +63,19 @@ struct __attribute__((aligned(G * sizeof(P)))) PcPack {
     P v[G];
 };
 
-// MFMA value-phase kernels (attention_mfma.hip): true if (D, G, mode) is
+// MFMA value-phase kernels (attn_mfma_kernel.h): true if (D, G, mode) is
 // handled there and the launch was issued.
 bool launch_mfma_split(int mode, int D, int G, const AttnArgs& a, dim3 grid, hipStream_t st, int nw = 4);
+// The instances of one head dim (one translation unit each, attn_mfma_d*.hip).
+template <int D>
+bool mfma_launch(int mode, int G, const AttnArgs& a, dim3 grid, hipStream_t st, int nw);
+template <int D>
+int mfma_occupancy(int mode, int G);
 // True if the MFMA kernels handle head_dim D with splits of `chunk` keys.
 bool mfma_split_ok(int D, int64_t chunk);
+// Head dims whose kernels append a token in place (the one-slice row encoder
+// of encode_row.h takes power-of-two lane groups).
+__host__ __device__ constexpr bool append_dim(int D) { return D == 64 || D == 128 || D == 256; }
 // Resident workgroups per CU of the MFMA kernel of (mode, D, G) on the current
 // device (0 when no MFMA kernel handles it).
 int mfma_wgs_per_cu(int mode, int D, int G);

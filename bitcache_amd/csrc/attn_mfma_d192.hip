@@ -1,0 +1,7 @@
+// The matrix-core attention kernels of head dim 192.
+#include "attn_mfma_kernel.h"
+
+namespace bc {
+template bool mfma_launch<192>(int, int, const AttnArgs&, dim3, hipStream_t, int);
+template int mfma_occupancy<192>(int, int);
+}  // namespace bc

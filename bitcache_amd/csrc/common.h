@@ -86,6 +86,14 @@ __device__ __forceinline__ float wave_max(float v) {
     const float b = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 32));
     return fmaxf(a, b);
 }
+// Max over the lane's half wave (32 lanes), in every lane of the half.
+__device__ __forceinline__ float half_max(float v) {
+    v = fmaxf(v, dpp_f<0x128>(v));
+    v = fmaxf(v, dpp_f<0x124>(v));
+    v = fmaxf(v, dpp_f<0x122>(v));
+    v = fmaxf(v, dpp_f<0x121>(v));
+    return fmaxf(v, swz_f<0x401F>(v));
+}
 __device__ __forceinline__ float wave_sum(float v) {
     v += dpp_f<0x128>(v);
     v += dpp_f<0x124>(v);
