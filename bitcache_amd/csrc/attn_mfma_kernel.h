@@ -151,7 +151,8 @@ struct WaveLds {
     // weight columns of 72 slots (64 used): the 16 lanes of a row group read
     // 16-byte runs of 16 columns without LDS bank conflicts
     static constexpr int kColSlots = 72;
-    static constexpr int kWeightBytes = 2 * 2 * G * kColSlots * 2;
+    // (one part where the int8 path holds the other)
+    static constexpr int kWeightBytes = (G <= 4 ? 1 : 2) * 2 * G * kColSlots * 2;
     static constexpr int kRdInts = KMF ? 64 * G : 4;
     // epilogue: heads per pass through staging buffer 0 ([parts][heads][D] floats)
     static constexpr int kEpiHeads = kStage / ((RES ? 2 : 1) * D * 4) < G ? kStage / ((RES ? 2 : 1) * D * 4) : G;
@@ -182,6 +183,11 @@ __device__ __forceinline__ v4i_t codes_i8(uint32_t x0, uint32_t x1) {
 __device__ __forceinline__ int opaque_int(int x) {
     asm volatile("" : "+v"(x));
     return x;
+}
+
+// a wave-uniform float, in a scalar register
+__device__ __forceinline__ float uniform_f(float f) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f)));
 }
 
 __device__ __forceinline__ uint16_t f2h_bits(float f) { return __builtin_bit_cast(uint16_t, (_Float16)f); }
@@ -427,10 +433,10 @@ template <int D, int G, int MODE>
 struct Occupancy {
     // Compensated heads above d = 128: two waves where the tile's operands fit
     // 256 registers with next to no spilling (one wave's latencies are
-    // exposed: 100 MB of cache, two against one: d = 256 MHA 39.7 / 60.9 us,
-    // groups of 2 30.4 / 33.9; d = 160 groups of 4 30.1 / 35.2), one where
-    // they do not (d = 256, groups of 4: 37.2 us at one, 56.9 at two)
-    static constexpr bool kTwo = G <= 2 || (G == 4 && D <= 192) || D <= 160;
+    // exposed: 100 MB of cache, two against one: d = 256 MHA 38 / 61 us,
+    // groups of 2 29 / 34; d = 224 groups of 4 36.5 / 40.6), one where they
+    // do not (d = 256, groups of 4: 37.4 us at one, 47.0 at two)
+    static constexpr bool kTwo = G <= 2 || (G == 4 && D <= 224) || D <= 160;
     static constexpr int kWaves =
         MODE == MODE_BINARY     ? (D <= 128 ? (G <= 2 ? BC_BIN_WAVES : 3) : 2)
         : MODE == MODE_ADAPTIVE ? (D <= 128 ? BC_ADAPT_WAVES : 1)
@@ -501,26 +507,45 @@ void attn_mfma_kernel(AttnArgs a) {
                           (MODE == MODE_ADAPTIVE && BC_ADAPT_PIPE) || BC_GQA_PIPE;
     using WL = WaveLds<D, G, RES, KMF>;
     using KR = KRegs<D, KMF>;
-    // Binary and adaptive modes, groups up to 4: the sign-part value MFMAs
-    // run on int8 operands (the residual part keeps fp16).  The sign bits
-    // enter in place (element 2^p for bit p of a nibble, four keys per AND
-    // instead of two fp16 elements) and each weight as an integer below 2^22
-    // in three balanced 8-bit digit columns (columns 4g + plane, the fourth
-    // unused), summed exactly in int32 accumulators.  A rescale (running max
-    // or weight plan) flushes those sums, scaled, into a per-wave float bank
-    // in LDS and restarts them at zero (flush8).
-    constexpr bool I8 = (MODE == MODE_BINARY || MODE == MODE_ADAPTIVE) && G <= 4;
-    constexpr int kW8Stride = 80;   // bytes per int8 weight column (64 slots + pad)
+    // Groups up to 4: the sign-part value MFMAs run on int8 operands.  The
+    // sign bits enter in place (element 2^p for bit p of a nibble, four keys
+    // per AND instead of two fp16 elements) and each weight as an integer up
+    // to 2^30 in four balanced 8-bit digit columns (columns 4g + j): the bytes
+    // of w + 0x80808080, each less 128, so two operations give the packed
+    // word.  The sums are exact in int32 accumulators.  A rescale (running max
+    // or weight plan) flushes them, scaled, into a per-wave float bank in LDS
+    // and restarts them at zero (flush8).
+    // R8: the residual part too (every mode but adaptive, whose residual
+    // positions are compacted): a code n enters as 16 n, eight codes in three
+    // operations, its weight as digits of the same kind, and no offset is
+    // needed for the codes' sign (fp16 codes are n + 8).  The sums are exact,
+    // where fp32 accumulation in the matrix cores drops low bits of every
+    // partial sum (the fp16 path at unit variance: 2.6e-4 to 2.9e-4 of the
+    // output against 64 bits; the fp16 output's own rounding is 2.1e-4).
+    constexpr bool I8 = G <= 4;
+    constexpr bool R8 = I8 && ALLRES;
+    // int8 weights in LDS: a row per slot, 4 digit bytes per head (and part),
+    // read back as columns by ds_read_b64_tr_b8 (16-byte rows; a shorter row
+    // is read twice, its columns repeating).  Up to two heads, one row holds
+    // the sign weights then the residual weights, so one operand serves both
+    // parts; four heads take two 16-byte halves.
+    constexpr int kWRow = G == 4 ? (R8 ? 32 : 16) : (G == 2 && R8 ? 16 : 8);
+    constexpr int kResCol = (R8 && G <= 2) ? 4 * G : 0;   // first residual digit column
+    // tiles whose sums int32 holds: a residual digit adds at most
+    // 128 * 112 * 64 < 2^20 per tile
+    constexpr int kMaxTiles8 = 2000;
 
     __shared__ QDigits<D, G, KMF> qd;
-    __shared__ __attribute__((aligned(16))) float qf[G * D];
     __shared__ __attribute__((aligned(16))) uint8_t lds_st0[NW][WL::kStage];
     __shared__ __attribute__((aligned(16))) uint8_t lds_st1[NW][PIPE ? WL::kStage : 16];
-    __shared__ __attribute__((aligned(16))) uint16_t lds_wts[NW][(I8 && !RES) ? 8 : WL::kWeightBytes / 2];
-    __shared__ __attribute__((aligned(16))) int8_t lds_w8[NW][I8 ? 4 * G * kW8Stride : 16];
+    __shared__ __attribute__((aligned(16))) uint16_t lds_wts[NW][(I8 && MODE != MODE_ADAPTIVE) ? 8 : WL::kWeightBytes / 2];
+    __shared__ __attribute__((aligned(16))) uint8_t lds_w8[NW][I8 ? 64 * kWRow : 16];
     // (int8 path) per wave and head, the float sums of the keys before the
-    // last rescale, [head][D] in the epilogue's dim order
+    // last rescale, [head][D]
     __shared__ __attribute__((aligned(16))) float lds_bank[NW][I8 ? G * D : 4];
+    // the query as floats during its preparation (the bank is free until then)
+    __shared__ __attribute__((aligned(16))) float lds_qf[I8 ? 4 : G * D];
+    float* const qf = I8 ? &lds_bank[0][0] : lds_qf;
     __shared__ __attribute__((aligned(16))) int lds_rd[NW][WL::kRdInts];
     __shared__ __attribute__((aligned(16))) int lds_rdlo[NW][(KMF && G > 1 && 3 * G <= 16) ? WL::kRdInts : 1];
     __shared__ float wofs[NW][G];
@@ -754,10 +779,9 @@ void attn_mfma_kernel(AttnArgs a) {
 
     // weight column owned by this lane in the MFMA B operand, and its head
     const int my_col = lj;
-    // (int8 path: the sign part's columns are 4 per head, the residual
-    // part's 2 per head as in the fp16 layout)
-    const int my_head = I8 ? my_col >> 2 : my_col >> 1;
-    const int my_rhead = my_col >> 1;
+    // (int8 columns: 4 per head, repeating past the last; fp16: 2 per head)
+    const int my_head = I8 ? (my_col >> 2) % G : my_col >> 1;
+    const int my_rhead = R8 ? my_head : my_col >> 1;
     const int bcol = my_col < 2 * G ? my_col : (my_col & 1);
 
     // weight columns [2 parts][2G cols][72 slots]: this lane's store slot in
@@ -767,20 +791,18 @@ void attn_mfma_kernel(AttnArgs a) {
     // tie to one array wait for all direct loads in flight, the prefetch too)
     uint16_t* wsl = &lds_wts[0][0] + opaque_int(wave * (WL::kWeightBytes / 2) + slot_of(kown));
     const uint16_t* wrd = &lds_wts[0][0] + opaque_int(wave * (WL::kWeightBytes / 2) + bcol * WL::kColSlots + 16 * g4);
-    // int8 weight columns [4G cols][80 bytes]: this lane's digit bytes at its
-    // key's slot of column 0, and its B-operand read (16 bytes of column
-    // my_col; lanes of unused columns read column 0 again)
-    int8_t* w8st = &lds_w8[0][0] + opaque_int(wave * (I8 ? 4 * G * kW8Stride : 16) + (I8 ? slot8_of(kown) : 0));
-    const int8_t* w8rd = &lds_w8[0][0] + opaque_int(wave * (I8 ? 4 * G * kW8Stride : 16) +
-                                                    (I8 ? (my_col < 4 * G ? my_col : 0) * kW8Stride + 16 * g4 : 0));
+    // int8 weights: this lane's key's row, and the row halves it reads for the
+    // sign and residual operands (slots 16 g4 + 0..7; the next eight follow)
+    uint8_t* w8st = &lds_w8[0][0] + opaque_int(I8 ? (wave * 64 + slot8_of(kown)) * kWRow : 0);
+    const uint8_t* w8rd = &lds_w8[0][0] + opaque_int(I8 ? (wave * 64 + 16 * g4 + (lj >> 1)) * kWRow + (kWRow >= 16 ? 8 * (lj & 1) : 0) : 0);
     int* rdl = lds_rd[wave];          // [64 keys][G] residual dots
     int* rdlo = lds_rdlo[wave];       // their plane-0 parts (precise tiles)
 
+    constexpr int kRes0 = I8 ? 0 : 2 * G;   // first fp16 residual weight column
     // softmax reference per head, lowered lazily: weights p = 2^(s - m) stay
     // <= 2^kTau, and the accumulators are rescaled only when a score passes
-    // m + kTau (the result does not depend on m).  The int8 path's fixed-point
-    // weights give up kTau of their 22 bits to this headroom: 4 there.
-    constexpr int kTauI = I8 ? 4 : 8;
+    // m + kTau (the result does not depend on m)
+    constexpr int kTauI = 8;
     constexpr float kTau = (float)kTauI;
     float m[G], mlim[G], lsum[G], off[G];
 #pragma unroll
@@ -792,7 +814,8 @@ void attn_mfma_kernel(AttnArgs a) {
     }
     f4_t cs[I8 ? 1 : NH][4];   // sign part: [block][p] rows = dims 64h + 4m + p
     v4i_t ci[I8 ? NH : 1][4];  // (int8 path) the same, per digit column
-    f4_t cn[NB];      // residual part: rows = dims 16db + m
+    f4_t cn[R8 ? 1 : NB];      // residual part: rows = dims 16db + m
+    v4i_t cr[R8 ? NB : 1];     // (int8 path) the same, per digit column
 #pragma unroll
     for (int h = 0; h < (I8 ? 1 : NH); h++)
 #pragma unroll
@@ -802,25 +825,43 @@ void attn_mfma_kernel(AttnArgs a) {
 #pragma unroll
         for (int p = 0; p < 4; p++) ci[h][p] = v4i_t{0, 0, 0, 0};
 #pragma unroll
-    for (int d = 0; d < NB; d++) cn[d] = f4_t{0.f, 0.f, 0.f, 0.f};
+    for (int d = 0; d < (R8 ? 1 : NB); d++) cn[d] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < (R8 ? NB : 1); d++) cr[d] = v4i_t{0, 0, 0, 0};
 
-    // (int8 path) a head's digit columns 4g + 0..2 are one lane quad; its
-    // first lane owns the head's rows in the bank.  flush8: bank = (bank +
-    // d0 + 256 d1 + 65536 d2) * f per element, the integer sums restart at 0
+    // (int8 path) a head's digit columns are one lane quad; the quad's first
+    // lane owns the head's rows.  digits(): d0 + 256 d1 + 65536 d2 + 2^24 d3
+    // of the quad (each lane scales its own digit, then a quad sum)
     const bool owner8 = I8 && my_col < 4 * G && (my_col & 3) == 0;
-    float* bank = &lds_bank[0][0] + opaque_int(wave * (I8 ? G * D : 4) + (I8 ? (my_col >> 2) * D : 0));
+    const bool rowner8 = R8 && my_col >= kResCol && my_col < kResCol + 4 * G && (my_col & 3) == 0;
+    auto digits = [&](int c, float dscale) {
+        float v = (float)c * dscale;
+        v += dpp_f<0xB1>(v);
+        return v + dpp_f<0x4E>(v);
+    };
+    // the lane's factor 256^digit (formed where it is used: one register less
+    // in the tile loop)
+    auto digit_scale = [&] {
+        return __builtin_bit_cast(float, 0x3F800000u + ((uint32_t)(opaque_int(lane) & 3) << 26));
+    };
+    // flush8: bank = (bank + integer sums) * f, the integer sums restart at 0
+    auto bank_at = [&] {
+        return &lds_bank[0][0] + (I8 ? (wave * G + ((opaque_int(lane) & 15) >> 2) % G) * D : 0);
+    };
     bool banked = false;   // (wave-uniform) the bank holds values
-    bool live8 = false;    // (wave-uniform) the integer sums hold values
+    int live8 = 0;         // (wave-uniform) tiles in the integer sums
     auto flush8 = [&](float f) {
+        const float dscale = digit_scale();
+        float* const bank = bank_at();
 #pragma unroll
         for (int h = 0; h < NH; h++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
+                // (accumulator p carries 2^p: bit p read in place)
                 float t[4];
 #pragma unroll
                 for (int p = 0; p < 4; p++) {
-                    const float v0 = (float)ci[h][p][i];
-                    t[p] = v0 + 256.0f * dpp_f<0x39>(v0) + 65536.0f * dpp_f<0x4E>(v0);
+                    t[p] = digits(ci[h][p][i], dscale) * (1.0f / (float)(1 << p));
                     ci[h][p][i] = 0;
                 }
                 if (owner8 && (64 * h + 16 * g4 < D)) {
@@ -829,14 +870,35 @@ void attn_mfma_kernel(AttnArgs a) {
                     *bp = make_float4((b.x + t[0]) * f, (b.y + t[1]) * f, (b.z + t[2]) * f, (b.w + t[3]) * f);
                 }
             }
+        if constexpr (R8) {
+            // (codes as 16 n)
+#pragma unroll
+            for (int d = 0; d < NB; d++) {
+                float t[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    t[i] = digits(cr[d][i], dscale) * (1.0f / 16.0f);
+                    cr[d][i] = 0;
+                }
+                if (rowner8) {
+                    float4* bp = (float4*)&bank[16 * d + 4 * g4];
+                    const float4 b = *bp;
+                    *bp = make_float4(b.x + t[0] * f, b.y + t[1] * f, b.z + t[2] * f, b.w + t[3] * f);
+                }
+            }
+        }
         banked = true;
+        live8 = 0;
     };
 
     // weights enter the MFMAs as w * 2^wexp (fp16 hi + lo), wexp chosen so the
-    // largest possible weight sits near 2^14 (int8 path: integers up to 2^22):
+    // largest possible weight sits near 2^14 (int8 path: integers up to 2^30):
     // no overflow, and weights down to ~2^-30 of the largest keep their
-    // contribution (fp16; undone exactly in the epilogue)
-    constexpr int kWTop = I8 ? 22 : 14;
+    // contribution (fp16; undone exactly in the epilogue).  The int8 path
+    // plans for value scales twice the largest seen, since lowering its plan
+    // costs a flush.
+    constexpr int kWTop = I8 ? 30 : 14;
+    constexpr int kSlack = I8 ? 1 : 0;
     int wexp = 0;
     bool have_wexp = false;
     float wlim = 0.0f;
@@ -866,7 +928,9 @@ void attn_mfma_kernel(AttnArgs a) {
     // (uniform operands of v_dot8) when codes are read per key, and the int8
     // MFMA B operands of the K residual dot (loop invariant)
     int sdig[(G == 1 && RES && !LIN_K) ? CW : 1][4];
-    v4i_t bq[KMF ? KB::kMfma : 1];
+    // (groups of four and more: read per tile, their registers are full)
+    constexpr bool BQ_LDS = KMF && ALLRES && G >= 4;
+    v4i_t bq[KMF && !BQ_LDS ? KB::kMfma : 1];
     if constexpr (G == 1 && RES && !LIN_K) {
 #pragma unroll
         for (int w = 0; w < CW; w++) {
@@ -877,7 +941,7 @@ void attn_mfma_kernel(AttnArgs a) {
             sdig[w][3] = __builtin_amdgcn_readfirstlane(dg.w);
         }
     }
-    if constexpr (KMF) {
+    if constexpr (KMF && !BQ_LDS) {
 #pragma unroll
         for (int m = 0; m < KB::kMfma; m++) {
             const int4 w = qd.bq[m][lane];
@@ -1044,6 +1108,13 @@ void attn_mfma_kernel(AttnArgs a) {
             // bits of the sum; smaller groups have it in rows 2G + g (below)
             constexpr bool LO_COLS = 3 * G <= 16;
             v4i_t acc[4];
+            v4i_t bt[KB::kMfma];   // this tile's B operands
+            const int lz = BQ_LDS ? opaque_int(lane) : 0;   // (read per tile, not hoisted)
+#pragma unroll
+            for (int m = 0; m < KB::kMfma; m++) {
+                if constexpr (BQ_LDS) bt[m] = *(const v4i_t*)&qd.bq[m][lz];
+                else bt[m] = bq[m];
+            }
 #pragma unroll
             for (int kb = 0; kb < 4; kb++) {
                 if (kb >= nkb) break;
@@ -1052,7 +1123,7 @@ void attn_mfma_kernel(AttnArgs a) {
 #pragma unroll
                 for (int m = 0; m < KB::kMfma; m++) {
                     const v4i_t av = codes_i8(kc[kb * KB::kWords + 2 * m], kc[kb * KB::kWords + 2 * m + 1]);
-                    acc[kb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bq[m], av, acc[kb], 0, 0, 0);
+                    acc[kb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bt[m], av, acc[kb], 0, 0, 0);
                     if (!LO_COLS && prec) {
                         const int4 w = qd.bq_lo[m][lane];
                         accl = __builtin_amdgcn_mfma_i32_16x16x64_i8(v4i_t{w.x, w.y, w.z, w.w}, av, accl, 0, 0, 0);
@@ -1247,7 +1318,7 @@ void attn_mfma_kernel(AttnArgs a) {
             if (__ballot(wb > wlim) != 0ull) {
                 const float wmx = wave_max(wb);
                 if (wmx < INFINITY) {
-                    const int e = kWTop - kTauI - (int)ceilf(log2f(wmx));
+                    const int e = kWTop - kTauI - kSlack - (int)ceilf(log2f(wmx));
                     if (have_wexp) {
                         // a larger weight than planned (e < wexp): bring the sums down
                         const float f = ldexpf(1.0f, e - wexp);
@@ -1259,8 +1330,10 @@ void attn_mfma_kernel(AttnArgs a) {
 #pragma unroll
                                 for (int p = 0; p < 4; p++) cs[h][p] *= f;
                         }
+                        if constexpr (!R8) {
 #pragma unroll
-                        for (int d = 0; d < NB; d++) cn[d] *= f;
+                            for (int d = 0; d < NB; d++) cn[d] *= f;
+                        }
 #pragma unroll
                         for (int g = 0; g < G; g++) off[g] *= f;
                     }
@@ -1280,25 +1353,31 @@ void attn_mfma_kernel(AttnArgs a) {
         // (the residual row of a key is its compacted position's row, of the
         // parity of rpos); the int8 sign elements carry no such factor
         const float kfac = (!I8 && (kown & 1)) ? 0.0625f : 1.0f;
-        const float kfac_res = (rpos & 1) ? 0.0625f : 1.0f;
+        const float kfac_res = (!R8 && (rpos & 1)) ? 0.0625f : 1.0f;
         // per-key factors shared by the heads: sign weight a2 = p * fa, residual
         // weight b = p * fb, and the offset sum_s (a_s + 8 b_s) grows by p * fo
         const float fa = ldexpf(2.0f * svv * kfac, wexp);
-        // (int8 path: the fp16 residual weights stay below 2^14 at 2^(wexp - 8))
-        const float fb = RES ? ldexpf(rsv * (1.0f / 7.0f) * kfac_res, wexp - (kWTop - 14)) : 0.0f;
+        // (adaptive: the fp16 residual weights stay below 2^14 at 2^(wexp - 16))
+        const float fb = RES ? ldexpf(rsv * (1.0f / 7.0f) * kfac_res, wexp - (R8 ? 0 : kWTop - 14)) : 0.0f;
         const float fo_bin = ldexpf(svv, wexp);
-        const float fo_res = RES ? ldexpf(svv + rsv * (8.0f / 7.0f), wexp) : fo_bin;
+        // (int8 codes need no offset; a V scale that is not finite has no
+        // integer weight, and makes the offset, so the output, NaN)
+        const float fo_res = R8 ? fmaf(svv + rsv, 0.0f, fo_bin) : RES ? ldexpf(svv + rsv * (8.0f / 7.0f), wexp) : fo_bin;
         // residual weights go to the slot of the key's residual position
         // (adaptive: compacted; unselected keys write zeros to the positions
         // past nsel, so every slot a residual MFMA reads is written)
         uint16_t* wres = wsl;
+        uint32_t dsig[G], dres[G];   // (int8 path) packed digits
+        // the weight p * f <= 2^30, rounded (weights are not negative), as
+        // balanced digits
+        auto pack8 = [](float p, float f) { return ((uint32_t)(int)fmaf(p, f, 0.5f) + 0x80808080u) ^ 0x80808080u; };
         if constexpr (MODE == MODE_ADAPTIVE)
             wres = &lds_wts[0][0] + opaque_int(wave * (WL::kWeightBytes / 2) + slot_of(res_row(rpos)));
 #pragma unroll
         for (int g = 0; g < G; g++) {
             // the reference m[g] moves only when a score passes m[g] + kTau
             if (__ballot(sc[g] > mlim[g]) != 0ull) {
-                const float mn = fmaxf(m[g], wave_max(sc[g]));
+                const float mn = uniform_f(fmaxf(m[g], wave_max(sc[g])));
                 const float alpha = __builtin_amdgcn_exp2f(m[g] - mn);   // 0 when m was -inf
                 lsum[g] *= alpha;
                 off[g] *= alpha;
@@ -1311,55 +1390,49 @@ void attn_mfma_kernel(AttnArgs a) {
             const float p = valid ? __builtin_amdgcn_exp2f(sc[g] - m[g]) : 0.0f;
             lsum[g] += p;
             const float a2 = p * fa;
-            float bv = 0.0f, fo = fo_bin;
-            if constexpr (MODE == MODE_COMP) {
-                bv = p * fb;
-                fo = fo_res;
-            }
-            if constexpr (MODE == MODE_MIXED) {
-                bv = hmode[g] ? p * fb : 0.0f;
-                fo = hmode[g] ? fo_res : fo_bin;
-            }
-            if constexpr (MODE == MODE_ADAPTIVE) {
-                const bool selg = (selmask >> g) & 1u;
-                bv = selg ? p * fb : 0.0f;
-                fo = selg ? fo_res : fo_bin;
-            }
+            bool with_res = MODE == MODE_COMP;   // the head takes the key's residual
+            if constexpr (MODE == MODE_MIXED) with_res = hmode[g];
+            if constexpr (MODE == MODE_ADAPTIVE) with_res = (selmask >> g) & 1u;
+            const float bv = with_res ? p * fb : 0.0f;
+            const float fo = with_res ? fo_res : fo_bin;
             // offset removed at the end, from the unrounded weights: the (hi, lo)
             // pairs carry ~22 bits (int8 path: rounding to integers up to
-            // 2^22), so the difference is a zero-mean ~2^-22 term
+            // 2^30), so the difference is a zero-mean term below 2^-22
             off[g] = fmaf(p, fo, off[g]);
             if constexpr (I8) {
-                // w = rint(a2) <= 2^22 from the low mantissa bits of
-                // a2 + 1.5 * 2^23, as balanced digits d0 + 256 d1 + 65536 d2:
-                // the bytes of w, of (w + 128) >> 8 and of (w + 32896) >> 16
-                const uint32_t wb3 = __builtin_bit_cast(uint32_t, a2 + 12582912.0f);
-                int8_t* ws = w8st + 4 * g * kW8Stride;
-                ws[0] = (int8_t)wb3;
-                ws[kW8Stride] = (int8_t)((wb3 + 128u) >> 8);
-                ws[2 * kW8Stride] = (int8_t)((wb3 - 4161408u) >> 16);   // (0x4B400000 - 0x400000 + 32896)
+                dsig[g] = pack8(p, fa);
             } else {
                 const uint16_t a2h = f2h_bits(a2);
                 const uint16_t a2l = f2h_bits(a2 - h_bits2f(a2h));
                 wsl[(0 * 2 * G + 2 * g) * WL::kColSlots] = a2h;
                 wsl[(0 * 2 * G + 2 * g + 1) * WL::kColSlots] = a2l;
             }
-            if constexpr (RES) {
+            if constexpr (R8) {
+                dres[g] = pack8(p, with_res ? fb : 0.0f);
+            } else if constexpr (RES) {
                 const uint16_t bh = f2h_bits(bv);
                 const uint16_t bl = f2h_bits(bv - h_bits2f(bh));
-                wres[(1 * 2 * G + 2 * g) * WL::kColSlots] = bh;
-                wres[(1 * 2 * G + 2 * g + 1) * WL::kColSlots] = bl;
+                wres[(kRes0 + 2 * g) * WL::kColSlots] = bh;
+                wres[(kRes0 + 2 * g + 1) * WL::kColSlots] = bl;
             }
+        }
+        if constexpr (I8 && G == 4) {
+            *(v4u_t*)w8st = v4u_t{dsig[0], dsig[1], dsig[2], dsig[3]};
+            if constexpr (R8) *(v4u_t*)(w8st + 16) = v4u_t{dres[0], dres[1], dres[2], dres[3]};
+        } else if constexpr (I8 && G == 2) {
+            if constexpr (R8) *(v4u_t*)w8st = v4u_t{dsig[0], dsig[1], dres[0], dres[1]};
+            else *(v2u_t*)w8st = v2u_t{dsig[0], dsig[1]};
+        } else if constexpr (I8) {
+            if constexpr (R8) *(v2u_t*)w8st = v2u_t{dsig[0], dres[0]};
+            else *(uint32_t*)w8st = dsig[0];
         }
         if constexpr (I8) {
             // the integer sums so far move to the float bank, scaled by this
-            // tile's factors (rare: the weight plan was lowered or a score
-            // passed m + kTau)
-            if (live8 && (any_rescale || wfac != 1.0f)) {
-                if (my_head >= G) lane_alpha = 1.0f;
+            // tile's factors (rare: the weight plan was lowered, a score
+            // passed m + kTau, or the residual sums are full)
+            if (live8 > 0 && (any_rescale || wfac != 1.0f || (R8 && live8 >= kMaxTiles8)))
                 flush8(lane_alpha * wfac);
-            }
-            if (RES && any_rescale) {
+            if (RES && !R8 && any_rescale) {
                 if (my_rhead >= G) lane_ralpha = 1.0f;
 #pragma unroll
                 for (int d = 0; d < NB; d++) cn[d] *= lane_ralpha;
@@ -1388,21 +1461,29 @@ void attn_mfma_kernel(AttnArgs a) {
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 
-        // B operands: (hi, lo) weight columns; lanes of unused columns read
-        // columns 0/1 again (their output columns are never read back)
+        // B operands: (hi, lo) weight columns (lanes of unused columns read
+        // columns 0/1 again, their output columns are never read back), or
+        // the digit columns of the int8 rows
         h8_t bsig[2], bres[2];
-        v4i_t b8 = v4i_t{0, 0, 0, 0};
+        v4i_t b8 = v4i_t{0, 0, 0, 0}, b8r = v4i_t{0, 0, 0, 0};
         if constexpr (I8) {
-            b8 = *(const v4i_t*)w8rd;
-            if constexpr (RES) {
+            auto columns = [&](const uint8_t* at) {
+                const v2i_t lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i_t, at));
+                const v2i_t hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32(LDS_PTR(v2i_t, at + 8 * kWRow));
+                return v4i_t{lo.x, lo.y, hi.x, hi.y};
+            };
+            b8 = columns(w8rd);
+            b8r = b8;
+            if constexpr (R8 && G == 4) b8r = columns(w8rd + 16);
+            if constexpr (RES && !R8) {
 #pragma unroll
-                for (int mh = 0; mh < 2; mh++) bres[mh] = *(const h8_t*)&wrd[(1 * 2 * G) * WL::kColSlots + 8 * mh];
+                for (int mh = 0; mh < 2; mh++) bres[mh] = *(const h8_t*)&wrd[kRes0 * WL::kColSlots + 8 * mh];
             }
         } else {
 #pragma unroll
             for (int mh = 0; mh < 2; mh++) {
-                bsig[mh] = *(const h8_t*)&wrd[(0 * 2 * G) * WL::kColSlots + 8 * mh];
-                if constexpr (RES) bres[mh] = *(const h8_t*)&wrd[(1 * 2 * G) * WL::kColSlots + 8 * mh];
+                bsig[mh] = *(const h8_t*)&wrd[8 * mh];
+                if constexpr (RES) bres[mh] = *(const h8_t*)&wrd[kRes0 * WL::kColSlots + 8 * mh];
                 else bres[mh] = bsig[mh];
             }
         }
@@ -1445,7 +1526,7 @@ void attn_mfma_kernel(AttnArgs a) {
                     ci[h][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, b8, ci[h][p], 0, 0, 0);
                 }
             }
-            live8 = true;
+            live8++;
         }
 #pragma unroll
         for (int h = 0; h < (I8 ? 0 : NH); h++) {
@@ -1490,6 +1571,12 @@ void attn_mfma_kernel(AttnArgs a) {
 #pragma unroll
                 for (int db = 0; db < NB; db++) res_mfma(db, mh);
             }
+        } else if constexpr (R8) {
+            // int8: the lane's 16 keys of dimension 16db + lj as bytes 16 n,
+            // in the sign part's slot order
+#pragma unroll
+            for (int db = 0; db < NB; db++)
+                cr[db] = __builtin_amdgcn_mfma_i32_16x16x64_i8(codes_i8((uint32_t)wrs[db].x, (uint32_t)wrs[db].y), b8r, cr[db], 0, 0, 0);
         } else if constexpr (RES) {
 #pragma unroll
             for (int db = 0; db < NB; db++) {
@@ -1587,67 +1674,48 @@ void attn_mfma_kernel(AttnArgs a) {
     // buffer 0 kEpiHeads at a time ([parts][kEpiHeads][D] floats per wave).
     constexpr int HP = WL::kEpiHeads;
     const float two24 = 16777216.0f;
+    // the wave's reference, sums and weight scale per head (published by the
+    // first barrier below)
 #pragma unroll
     for (int g = 0; g < G; g++) {
-        const float l_w = wave_sum(lsum[g]);
-        const float o_w = wave_sum(off[g]);
-        if (lane == 0) {
+        const float l_w = wave_sum63(lsum[g]);
+        const float o_w = wave_sum63(off[g]);
+        if (lane == 63) {
             wm[wave][g] = m[g];
             wlsum[wave][g] = l_w;
             wofs[wave][g] = o_w;
         }
     }
     if (lane == 0) wsc[wave] = ldexpf(1.0f, -wexp);
-    // per head: the maximum M over the waves, each wave's factor
-    // 2^(m_w - M) * 2^-wexp_w (0 for a wave without keys) and the total l
-    // (published by the first barrier of the head batches below)
-    __shared__ float mfac[NW][G], hsum[2][G];
-    __syncthreads();
-    if (threadIdx.x < G) {
-        const int g = threadIdx.x;
-        float M = -INFINITY;
-        for (int w = 0; w < NW; w++) M = fmaxf(M, wm[w][g]);
-        float lv = 0.0f;
-        for (int w = 0; w < NW; w++) {
-            const bool live = M != -INFINITY && wm[w][g] != -INFINITY;
-            const float f = live ? exp2f(wm[w][g] - M) : 0.0f;
-            mfac[w][g] = f * wsc[w];
-            if (live) lv += f * wlsum[w][g];
-        }
-        hsum[0][g] = M;
-        hsum[1][g] = lv;
-    }
     float* accw = (float*)lds_st0[wave];
+    const float dscale = digit_scale();
+    const float* const bank = bank_at();
     // hi + lo columns are adjacent lanes (col 2g, 2g+1); the even lane writes.
-    // int8 path: the digit columns 4g + 0..2 of a head are one lane quad; its
-    // first lane writes
-    const bool writer = I8 ? (my_col < 4 * G && (my_col & 3) == 0) : (my_col < 2 * G && (my_col & 1) == 0);
+    // int8 path: the digit columns of a head are one lane quad; its first
+    // lane writes
+    const bool writer = I8 ? owner8 : (my_col < 2 * G && (my_col & 1) == 0);
     // the sign part's unit: 2^-24 (fp16 subnormal elements) or 1 (int8)
     const float sunit = I8 ? 1.0f : two24;
     for (int g0 = 0; g0 < G; g0 += HP) {
         const int hs = my_head - g0;   // this lane's head slot in the batch
         const bool wr = writer && hs >= 0 && hs < HP;
-        // the residual part's writer (fp16 column layout in both paths)
+        // the residual part's writer (adaptive: in the fp16 column layout)
         const int rhs = my_rhead - g0;
-        const bool rwr = my_col < 2 * G && (my_col & 1) == 0 && rhs >= 0 && rhs < HP;
+        const bool rwr = (R8 ? rowner8 : my_col < 2 * G && (my_col & 1) == 0) && rhs >= 0 && rhs < HP;
         if (g0 > 0) __syncthreads();   // the previous batch has been read
         // hi + lo: the neighbour lane's column by DPP (quad_perm [1,0,3,2]),
         // all sums first, then the stores under one branch
         float sv[I8 ? 1 : NH][4][4];
         float nv[RES ? NB : 1][4];
         if constexpr (I8) {
-            // digits d0 + 256 d1 + 65536 d2 from lanes +0, +1, +2 of the quad
-            // (quad_perm [1,2,3,0] and [2,3,0,1]); one 64-dim block at a time
-            // (accumulator p carries 2^p: bit p read in place)
+            // one 64-dim block at a time (accumulator p carries 2^p: bit p
+            // read in place)
 #pragma unroll
             for (int h = 0; h < NH; h++) {
 #pragma unroll
                 for (int p = 0; p < 4; p++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float v0 = (float)ci[h][p][i];
-                        sv[0][p][i] = v0 + 256.0f * dpp_f<0x39>(v0) + 65536.0f * dpp_f<0x4E>(v0);
-                    }
+                    for (int i = 0; i < 4; i++) sv[0][p][i] = digits(ci[h][p][i], dscale);
                 if (wr && 64 * h + 16 * g4 < D) {
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
@@ -1658,7 +1726,7 @@ void attn_mfma_kernel(AttnArgs a) {
 #pragma unroll
                         for (int p = 0; p < 4; p++)
                             accw[(0 * HP + hs) * D + 64 * h + 4 * (4 * g4 + i) + p] =
-                                (sv[0][p][i] + bb[p]) * (1.0f / (float)(1 << p));
+                                sv[0][p][i] * (1.0f / (float)(1 << p)) + bb[p];
                     }
                 }
             }
@@ -1676,7 +1744,10 @@ void attn_mfma_kernel(AttnArgs a) {
 #pragma unroll
             for (int d = 0; d < NB; d++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) nv[d][i] = cn[d][i] + dpp_f<0xB1>(cn[d][i]);
+                for (int i = 0; i < 4; i++) {
+                    if constexpr (R8) nv[d][i] = digits(cr[d][i], dscale) * (1.0f / 16.0f);   // (codes as 16 n)
+                    else nv[d][i] = cn[d][i] + dpp_f<0xB1>(cn[d][i]);
+                }
         }
         if (wr) {
 #pragma unroll
@@ -1690,40 +1761,49 @@ void attn_mfma_kernel(AttnArgs a) {
             }
         }
         if constexpr (RES) {
-            // (int8 path: the residual part's units of 2^-24, its weights
-            // 2^-8 of the sign weights' scale, become the sign part's units)
+            // (adaptive: the residual part's units of 2^-24, its weights 2^-16
+            // of the sign weights' scale, become the sign part's units)
             if (rwr) {
 #pragma unroll
                 for (int d = 0; d < NB; d++)
 #pragma unroll
                     for (int i = 0; i < 4; i++)
-                        accw[(1 * HP + rhs) * D + 16 * d + 4 * g4 + i] = I8 ? nv[d][i] * (two24 * 256.0f) : nv[d][i];
+                        accw[(1 * HP + rhs) * D + 16 * d + 4 * g4 + i] = I8 && !R8 ? nv[d][i] * (two24 * 65536.0f) : nv[d][i];
             }
         }
         __syncthreads();
         const int nh = min(HP, G - g0);
         for (int i = threadIdx.x; i < nh * D; i += blockDim.x) {
             const int hs2 = i / D, e = i % D, g = g0 + hs2;
-            float accv = 0.0f;
+            // the maximum M over the waves, each wave's factor 2^(m_w - M)
+            // (0 for a wave without keys) and the total l
+            float mw[NW], M = -INFINITY;
+#pragma unroll
+            for (int w = 0; w < NW; w++) {
+                mw[w] = wm[w][g];
+                M = fmaxf(M, mw[w]);
+            }
+            float accv = 0.0f, L = 0.0f;
 #pragma unroll
             for (int w = 0; w < NW; w++) {
                 const float* aw = (const float*)lds_st0[w];
                 float v = aw[(0 * HP + hs2) * D + e];
                 if (RES) v += aw[(1 * HP + hs2) * D + e];
-                const float f = mfac[w][g];
-                accv += f == 0.0f ? 0.0f : (v * sunit - wofs[w][g]) * f;
+                const bool live = mw[w] != -INFINITY;
+                const float f = live ? __builtin_amdgcn_exp2f(mw[w] - M) : 0.0f;
+                accv += live && f != 0.0f ? (v * sunit - wofs[w][g]) * (f * wsc[w]) : 0.0f;
+                if (live) L += f * wlsum[w][g];
             }
             if (a.out != nullptr) {
                 // one split: the output itself, normalised as the merge of a
                 // single partial would (factor 1, sum l)
-                const float L = hsum[1][g];
                 a.out[(int64_t)(bhq0 + g) * D + e] = f2h(L > 0.0f ? accv * (1.0f / L) : 0.0f);
             } else {
                 float* dst = a.ws + ((int64_t)(bhq0 + g) * a.n_splits + split) * (D + 2);
                 dst[2 + e] = accv;
                 if (e == 0) {
-                    dst[0] = hsum[0][g];
-                    dst[1] = hsum[1][g];
+                    dst[0] = M;
+                    dst[1] = L;
                 }
             }
         }

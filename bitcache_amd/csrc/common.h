@@ -104,6 +104,17 @@ __device__ __forceinline__ float wave_sum(float v) {
     const float b = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 32));
     return a + b;
 }
+// Sum over the wave without LDS moves; valid in lane 63: each 16-lane row's
+// sum in its last lane, then row broadcasts into the rows after.
+__device__ __forceinline__ float wave_sum63(float v) {
+    v += dpp_f<0x111>(v);
+    v += dpp_f<0x112>(v);
+    v += dpp_f<0x114>(v);
+    v += dpp_f<0x118>(v);
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x142, 0xA, 0xF, false));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x143, 0xC, 0xF, false));
+    return v;
+}
 __device__ __forceinline__ int lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
 
 // Sign-word loaders: D/8 bytes per vector, returned as D/32 uint32 words.
