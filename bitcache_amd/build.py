@@ -33,6 +33,8 @@ HIP_SOURCES = [f"attn_mfma_d{d}.hip" for d in (256, 224, 192, 160, 128, 96, 64, 
 HIP_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # the first sixteen argument dwords of a kernel arrive in scalar registers
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
     "-I" + INCLUDE, "-I" + CSRC,
 ]
 

@@ -7,25 +7,25 @@
 // Score phase (lane = key): XNOR popcount of the sign words, and the INT4
 // residual dot directly on the stored two's-complement nibbles against the
 // query in 24-bit fixed point: six balanced int4 digits for v_dot8_i32_i4
-// (MHA) or three balanced int8 planes for an int8 MFMA (GQA groups), of which
-// a tile uses the top 16 bits unless a key's residual scale makes it a
-// precise tile.
+// (single heads) or three balanced int8 planes for an int8 MFMA (KMF below),
+// of which a tile uses the top 16 bits unless a key's residual scale makes it
+// a precise tile.
 //
-// Value phase: out[e] = sum_s a_s*(2*bit_se - 1) + b_s*(u_se - 8) with
-// a = p*sv, b = p*rs/7, u = n + 8.  The V tile (sign bytes and code bytes of
-// 64 keys) is copied to LDS with direct buffer loads, then ds_read_b64_tr_b4
-// transposes 16 keys x 16 nibbles per 16-lane group so that each lane holds
-// 16 keys of one dimension.  fp16 path: nibbles (u) and sign bits become
-// exact fp16 subnormals (value * 2^(j-24) for bit position j < 10) with one
-// mask per pair of keys, left in place (the power of two is folded into the
-// weights of odd keys and into the accumulator of bit p), and
-// v_mfma_f32_16x16x32_f16 accumulates dims x weight-columns, where the weight
-// columns are (hi, lo) fp16 splits of a and b for each query head of the
-// group; the fp32 accumulators are rescaled on running-max changes.  int8
-// path (the sign part of binary and adaptive attention, groups up to 4):
-// sign bits in place as int8 elements, four keys per mask, weights as
-// balanced 8-bit digit columns, exact int32 sums flushed into a float bank on
-// rescales (see I8 below).
+// Value phase: out[e] = sum_s a_s*(2*bit_se - 1) + b_s*n_se with a = p*sv,
+// b = p*rs/7.  The V tile (sign bytes and code bytes of 64 keys) is copied to
+// LDS with direct buffer loads, then ds_read_b64_tr_b4 transposes 16 keys x 16
+// nibbles per 16-lane group so that each lane holds 16 keys of one dimension.
+// int8 path (groups up to 4; I8 and R8 below): sign bits in place as int8
+// elements, codes as 16 n, four keys per operation, the weights of each head
+// as balanced 8-bit digit columns, v_mfma_i32_16x16x64_i8 with exact int32
+// sums, flushed into a float bank on rescales.  fp16 path (groups of 8, and
+// the adaptive mode's residuals): nibbles (u = n + 8, the 8 b_s taken off at
+// the end) and sign bits become exact fp16 subnormals (value * 2^(j-24) for
+// bit position j < 10) with one mask per pair of keys, left in place (the
+// power of two is folded into the weights of odd keys and into the
+// accumulator of bit p), and v_mfma_f32_16x16x32_f16 accumulates dims x weight
+// columns, (hi, lo) fp16 splits of a and b for each query head of the group;
+// the fp32 accumulators are rescaled on running-max changes.
 #pragma once
 
 #include <math.h>
@@ -183,6 +183,14 @@ __device__ __forceinline__ v4i_t codes_i8(uint32_t x0, uint32_t x1) {
 __device__ __forceinline__ int opaque_int(int x) {
     asm volatile("" : "+v"(x));
     return x;
+}
+
+// (scale_q * scale_k) * (2pc - d)  (src/xnor_dot.cuh:30), two rounded products
+// in every instance: a step that appends and a call that attends give the
+// same bits
+__device__ __forceinline__ float xnor_score(float scale_q, float scale_k, float mq) {
+#pragma clang fp contract(off)
+    return (scale_q * scale_k) * mq;
 }
 
 // a wave-uniform float, in a scalar register
@@ -390,20 +398,16 @@ __device__ void prep_digits(const uint16_t (&qpre)[NQ], QDigits<D, G, KMF>& qd, 
 //   BC_BIN_WAVES   the same for binary attention of groups up to 2 (5)
 //   BC_ADAPT_WAVES the same for adaptive attention up to d = 128 (2; its LDS
 //                  holds two workgroups per CU at d = 128)
-//   BC_LIN_K / BC_LIN_V  code tiles read as linear KiB runs (1) instead of per key
+//   BC_LIN_V       V code tiles read as linear KiB runs (1) instead of per key
 //   BC_MHA_PIPE / BC_ADAPT_PIPE / BC_GQA_PIPE  one-tile prefetch with two staging
 //                  buffers for MHA (1), adaptive (1) and GQA compensated (0: one
 //                  buffer keeps a third workgroup per CU) kernels
 //   BC_NT_AUX      cache policy of the loads that cover whole KiB runs (K and V
-//                  sign rows, the linear V code tile, the K code blocks of GQA
-//                  groups, linear K code rows): 2 = nontemporal (8-11% faster;
+//                  sign rows, the linear V code tile, the K code blocks): 2 = nontemporal (8-11% faster;
 //                  lines that several loads share keep the default policy)
 //   BC_NT_SCALES   cache policy of the 2-byte scale loads (0: default)
 #ifndef BC_MHA_WAVES
 #define BC_MHA_WAVES 3
-#endif
-#ifndef BC_LIN_K
-#define BC_LIN_K 1
 #endif
 #ifndef BC_LIN_V
 #define BC_LIN_V 1
@@ -444,51 +448,57 @@ struct Occupancy {
                                 : (D <= 128 ? (G <= 4 && !BC_GQA_PIPE ? 3 : 2) : (kTwo ? 2 : 1));
 };
 
-// Sum of v over the Q consecutive lanes that share one key row (DPP, no LDS).
-template <int Q>
-__device__ __forceinline__ int row_group_sum(int v) {
-    if constexpr (Q >= 2) v += __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);   // quad_perm [1,0,3,2]
-    if constexpr (Q >= 4) v += __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true);   // quad_perm [2,3,0,1]
-    if constexpr (Q >= 8) v += __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true);  // row_half_mirror
-    return v;
-}
-
-// The K residual dots come from int8 MFMAs (see the kernel).
-__host__ __device__ constexpr bool k_on_mfma(int D, int G, int mode) {
-    const int q = D / 32;
-    return mode != MODE_BINARY && (G > 1 || (mode != MODE_ADAPTIVE && (q & (q - 1)) != 0));
+// The K residual dots come from int8 MFMAs (see the kernel): every instance
+// but the adaptive mode's single heads.
+__host__ __device__ constexpr bool k_on_mfma(int G, int mode) {
+    return mode != MODE_BINARY && (G > 1 || mode != MODE_ADAPTIVE);
 }
 
 // NW waves per workgroup (4, or 8 to 16 for a wide workgroup that takes all
 // keys of its group: one split, no merge launch); wave w takes tiles w, w + NW,
 // w + 2 NW, ... of the key range, and the epilogue merges the NW waves.
-template <int D, int G, int MODE, int NW = 4>
+// APP: the workgroup whose key range holds the slot a.app_slot appends the
+// token a.app_k / a.app_v there.
+//
+// The scalar arguments (14 dwords) come in registers with the wave (kernarg
+// preloading: a launch's first read of its argument memory takes about a
+// microsecond), so they are what the first loads' addresses need: the planes'
+// bases (each blob's scales follow its signs or codes, whose capacity is
+// kv_rows * kv_stride vectors) and the key range; plan packs the split's tiles
+// (bits 0..16), whether the launch's groups come from a list (bit 17) and the
+// head groups per kv head (bits 18..30).  Measured with it: one 64-key call
+// 0.9 us less.
+constexpr int kPlanList = 1 << 17, kPlanGroups = 18, kMaxHeadGroups = (1 << 13) - 1;
+inline int pack_plan(const AttnArgs& a, int G) {
+    return a.chunk / 64 | (a.group_list != nullptr ? kPlanList : 0) | (((a.Hq / a.Hkv) / G) << kPlanGroups);
+}
+#define BC_MFMA_ARGS(a, G)                                                                       \
+    (a).q, (a).kb.signs, (a).vb.signs, (a).kr.codes, (a).vr.codes, (a).B * (a).Hkv, (a).S,       \
+        (a).kv_stride, pack_plan(a, G), (a)
+template <int D, int G, int MODE, int NW = 4, bool APP = false>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(Occupancy<D, G, MODE>::kWaves)))
-void attn_mfma_kernel(AttnArgs a) {
+void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* v_signs,
+                      const uint8_t* k_codes, const uint8_t* v_codes, int kv_rows, int S, int kv_stride,
+                      int plan, AttnArgs a) {
     constexpr int NB = D / 16;   // nibble dim-blocks (16 dims each)
     constexpr int NH = (D + 63) / 64;   // sign blocks (64 dims each; D % 64 == 32: half of the last)
     constexpr int CW = D / 8;    // code dwords per key
     constexpr bool RES = MODE != MODE_BINARY;
     constexpr int SB = D / 8;    // sign bytes per key
     constexpr int CB = D / 2;    // code bytes per key
-    // Code loads.  Per key (lane = key): lane l reads its key's row in 16-byte
-    // pieces, so one load touches 64 rows.  Linear: load round i, lane l takes
-    // the 16 bytes at i*1024 + 16*l of the tile (contiguous KiB), i.e. piece
-    // l%Q of key i*(64/Q) + l/Q; for K this needs a Q-lane reduction of the
-    // partial dots.  The adaptive mode gathers only selected keys' codes and
-    // always works per key.
+    // Code loads.  V codes: linear, load round i, lane l takes the 16 bytes at
+    // i*1024 + 16*l of the tile (contiguous KiB); the adaptive mode gathers
+    // only selected keys' rows.  K codes: in the key blocks of the int8 MFMAs
+    // (KBlocks), or (adaptive single heads) the lane's own key's row.
     // every key's residual data is read (compensated, and mixed per-head modes)
     constexpr bool ALLRES = MODE == MODE_COMP || MODE == MODE_MIXED;
     constexpr int Q = D / 32;    // 16-byte pieces per code row
     constexpr bool Q_POW2 = (Q & (Q - 1)) == 0;
     // KMF: the K residual dots of all G heads come from one set of int8 MFMAs
     // (keys x dims times dims x (head, digit plane)); the lane holds code
-    // pieces of 16 keys (KBlocks) instead of one key's row.  GQA groups, and
-    // single heads whose code row is not a power of two of pieces (the linear
-    // reads' row sums need one)
-    constexpr bool KMF = k_on_mfma(D, G, MODE);
+    // pieces of 16 keys (KBlocks) instead of one key's row
+    constexpr bool KMF = k_on_mfma(G, MODE);
     using KB = KBlocks<D>;
-    constexpr bool LIN_K = BC_LIN_K && ALLRES && !KMF;
     constexpr bool LIN_V = BC_LIN_V && ALLRES;
     // Vector-memory operations issued per prefetched tile, counted at their
     // fewest (a load moves at most 16 bytes; planes are separate loads), so
@@ -552,32 +562,30 @@ void attn_mfma_kernel(AttnArgs a) {
     __shared__ float wm[NW][G], wlsum[NW][G], wsc[NW];
 
     const int split = blockIdx.x;
-    const int nqg = (a.Hq / a.Hkv) / G;
     // per-head modes: this launch's query-head groups come from its list
     int grow = blockIdx.y;
     if constexpr (MODE == MODE_BINARY || MODE == MODE_MIXED) {
-        if (a.group_list != nullptr) {
+        if (plan & kPlanList) {
             if (grow >= *a.group_count) return;
             grow = a.group_list[grow];
         }
     }
-    const int qg = grow % nqg;
+    // groups are numbered through batches, kv heads and the groups of a kv head
+    const int nqg = plan >> kPlanGroups;
     const int bkv = grow / nqg;
-    const int b = bkv / a.Hkv, kvh = bkv % a.Hkv;
-    const int hq0 = kvh * (a.Hq / a.Hkv) + qg * G;
-    const int bhq0 = b * a.Hq + hq0;
+    const int bhq0 = grow * G;   // first query head
+    const int64_t cap = (int64_t)kv_rows * kv_stride;
 
     // the wave index is uniform: readfirstlane lets the compiler keep the tile
     // loop in scalar registers (a uniform loop, not an exec-masked one)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int g4 = lane >> 4, lj = lane & 15;
-    const int key_begin = split * a.chunk;
-    const int key_end = min(a.S, key_begin + a.chunk);
-    const int64_t kv_base = (int64_t)bkv * a.kv_stride;
+    const int chunk = (plan & (kPlanList - 1)) * 64;
+    const int key_begin = split * chunk;
+    const int key_end = min(S, key_begin + chunk);
+    const int64_t kv_base = (int64_t)bkv * kv_stride;
     const float isd2 = (1.0f / sqrtf((float)D)) * kLog2e;
-    // the key whose score this lane computes (tile-relative)
-    const int kown = LIN_K ? (lane % Q) * (64 / Q) + lane / Q : lane;
-    const int quarter = lane % Q;
+    const int kown = lane;   // the key whose score this lane computes (tile-relative)
     // V code tiles of compensated mode (linear rows of CB bytes): the 16-byte
     // pieces of row k are stored at piece ^ vsw(k), vsw(k) = (k*CB/256) mod Q,
     // so the rows that one transposed read covers spread over the LDS banks;
@@ -595,16 +603,16 @@ void attn_mfma_kernel(AttnArgs a) {
         return __builtin_amdgcn_make_buffer_rsrc(
             (void*)((const uint8_t*)plane + (kv_base + key_begin) * rb), (short)0, nk * rb, kBufWord3);
     };
-    const __amdgpu_buffer_rsrc_t r_ks = rsrc(a.kb.signs, SB), r_vs = rsrc(a.vb.signs, SB);
-    const __amdgpu_buffer_rsrc_t r_ksc = rsrc(a.kb.scales, 2), r_vsc = rsrc(a.vb.scales, 2);
-    const __amdgpu_buffer_rsrc_t r_kc = rsrc(a.kr.codes, CB), r_vc = rsrc(a.vr.codes, CB);
-    const __amdgpu_buffer_rsrc_t r_krs = rsrc(a.kr.scales, 2), r_vrs = rsrc(a.vr.scales, 2);
+    const __amdgpu_buffer_rsrc_t r_ks = rsrc(k_signs, SB), r_vs = rsrc(v_signs, SB);
+    const __amdgpu_buffer_rsrc_t r_ksc = rsrc(k_signs + cap * SB, 2), r_vsc = rsrc(v_signs + cap * SB, 2);
+    const __amdgpu_buffer_rsrc_t r_kc = rsrc(k_codes, CB), r_vc = rsrc(v_codes, CB);
+    const __amdgpu_buffer_rsrc_t r_krs = rsrc(k_codes + cap * CB, 2), r_vrs = rsrc(v_codes + cap * CB, 2);
     // adaptive: stored popcounts of this group, one pack of G per key
     using Pack = bc::PcPack<bc::PcT<D>, G>;
     constexpr int kPack = (int)sizeof(Pack);
     static_assert(kPack <= 16, "one load per pack");
     const __amdgpu_buffer_rsrc_t r_pc = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)((const Pack*)a.pcs + (int64_t)bhq0 / G * bc::pcs_stride(a.S) + key_begin), (short)0, nk * kPack, kBufWord3);
+        (void*)((const Pack*)a.pcs + (int64_t)grow * bc::pcs_stride(S) + key_begin), (short)0, nk * kPack, kBufWord3);
     // an offset past every range (the host keeps each range's bytes below
     // 2^31 - 4096): such a load returns zeros and moves no data
     constexpr int kOob = 0x7FFFF000;
@@ -670,15 +678,6 @@ void attn_mfma_kernel(AttnArgs a) {
                 // key block kb: key 16kb + l%16
 #pragma unroll
                 for (int kb = 0; kb < 4; kb++) load_kblock(r, kb, (tr + 16 * kb + lj) * CB);
-            } else {
-                // per key: the lane's own row; linear: piece i*1024 + 16l of the tile
-                const int base = LIN_K ? tr * CB + 16 * lane : kk * CB;
-#pragma unroll
-                for (int i = 0; i < Q; i++) {
-                    const v4u_t c = __builtin_amdgcn_raw_buffer_load_b128(r_kc, base + (LIN_K ? i * 1024 : 16 * i), 0,
-                                                                          LIN_K ? BC_NT_AUX : 0);
-                    r.kc[4 * i] = c[0]; r.kc[4 * i + 1] = c[1]; r.kc[4 * i + 2] = c[2]; r.kc[4 * i + 3] = c[3];
-                }
             }
         }
     };
@@ -718,24 +717,22 @@ void attn_mfma_kernel(AttnArgs a) {
     };
 
     // The query's elements are loaded first, then the wave's first tile
-    // (except in adaptive mode, whose first tile needs the selection, and in
-    // the workgroup that appends a token), and the query preparation runs
-    // while that tile is in flight: it waits only for the older query loads,
-    // and its barriers wait for LDS traffic only.
+    // (except in adaptive mode, whose first tile needs the selection), and the
+    // query preparation runs while that tile is in flight: it waits only for
+    // the older query loads, and its barriers wait for LDS traffic only.
     constexpr int NT = NW * 64;
     constexpr int NQ = (G * D + NT - 1) / NT;
     uint16_t qpre[NQ];
     {
-        const uint16_t* qb = a.q + (int64_t)bhq0 * D;
+        const uint16_t* qb = q + (int64_t)bhq0 * D;
 #pragma unroll
         for (int j = 0; j < NQ; j++) {
             const int i = (int)threadIdx.x + NT * j;
             qpre[j] = i < G * D ? qb[i] : (uint16_t)0;
         }
     }
-    const bool app_here = a.app_k != nullptr && a.app_slot >= key_begin && a.app_slot < key_end;
     int t = key_begin + wave * 64;
-    const bool early = MODE != MODE_ADAPTIVE && !app_here && t < key_end;
+    const bool early = MODE != MODE_ADAPTIVE && t < key_end;
     KR ka, kb;
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (MODE != MODE_ADAPTIVE) {
@@ -748,32 +745,92 @@ void attn_mfma_kernel(AttnArgs a) {
         issue_v(0, t_first);
     }
     __builtin_amdgcn_sched_barrier(0);
+    // the appended token's slice of this lane (lane groups 0 and 1: K and V;
+    // loaded by every wave, so that the wait for the query counts the same)
+    constexpr int AL = D / 8;
+    bc_v4u app_raw = {0u, 0u, 0u, 0u};
+    if constexpr (APP) {
+        app_raw = bc::load_row_slice((lane / AL == 1 ? a.app_v : a.app_k) + (int64_t)bkv * D, lane % AL);
+        __builtin_amdgcn_sched_barrier(0);
+    }
     prep_digits<D, G, KMF, RES, NT>(qpre, qd, qf);
 
-    // In-place append: the workgroup whose key range holds the new token's slot
-    // encodes the token's K and V vectors into the cache first (wave 0, lane
-    // groups 0 and 1, online-encode semantics: the residual against the fp32
-    // mean).  Its stores complete before the barrier, so its own tile loads see
-    // them; no other workgroup reads the slot's cache lines (key ranges are
-    // whole 64-key tiles, and the host appends only with one query-head group
-    // per kv head), and later launches see them as after a separate encode.
-    if constexpr (MODE != MODE_ADAPTIVE && bc::append_dim(D)) {
-        if (a.app_k != nullptr && a.app_slot >= key_begin && a.app_slot < key_end) {
-            if (wave == 0) {
-                constexpr int L = D / 8;
-                const int grp = lane / L, j = lane % L;
-                const bool is_v = grp == 1;
-                const uint16_t* src = (is_v ? a.app_v : a.app_k) + (int64_t)bkv * D;
-                const BinPlanes& bp = is_v ? a.vb : a.kb;
-                const ResPlanes& rp = is_v ? a.vr : a.kr;
-                // (the attention arguments hold the cache planes read-only)
-                const bc::EncodeDst dst{(uint8_t*)bp.signs, (uint16_t*)bp.scales,
-                                        RES ? (uint8_t*)rp.codes : nullptr, RES ? (uint16_t*)rp.scales : nullptr};
-                bc::encode_row<D, RES ? bc::ENC_FUSED_FP32 : bc::ENC_BINARY>(src, j, grp < 2, dst,
-                                                                            kv_base + a.app_slot);
-                __builtin_amdgcn_s_waitcnt(0);
+    // In-place append: the wave that takes the slot's tile encodes the token's
+    // K and V vectors (online-encode semantics: the residual against the fp32
+    // mean) into LDS and stores them from there.  Nothing waits for the
+    // stores: the wave's tile is loaded with the slot's old contents, and when
+    // it is processed the token's score parts and dots (formed here, as a
+    // tile's are) and its V row take their place.  No other wave reads the
+    // slot (the host appends only with one query-head group per kv head), and
+    // later launches see the token as after a separate encode.  (Encoding
+    // first and then loading the tile is three dependent memory round trips:
+    // 3 us of a 27 us step.)
+    struct Token {
+        uint32_t signs[2][D / 32];
+        uint32_t codes[2][D / 8];
+        uint16_t scale[2], rscale[2];
+        float mq[G];             // 2 popcount - d of K against each query head
+        int dot[G], dot_lo[G];   // K residual dots: planes 1 and 2, plane 0
+    };
+    __shared__ Token token[1];
+    int app_t0 = -1;   // (wave-uniform) the slot's tile, if it is this wave's
+    if constexpr (APP) {
+        static_assert(bc::append_dim(D) && MODE != MODE_ADAPTIVE && MODE != MODE_MIXED, "append");
+        const int slot = a.app_slot, tile = (slot - key_begin) >> 6;
+        if (slot >= key_begin && slot < key_end && tile % NW == wave) {
+            app_t0 = key_begin + 64 * tile;
+            const int grp = lane / AL;
+            const int kv = grp == 1;
+            const bc::EncodeDst dst{(uint8_t*)token->signs[kv], &token->scale[kv],
+                                    RES ? (uint8_t*)token->codes[kv] : nullptr, &token->rscale[kv]};
+            bc::encode_row_slice<D, RES ? bc::ENC_FUSED_FP32 : bc::ENC_BINARY>(app_raw, lane % AL, grp < 2, dst, 0);
+            __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            if (lane < G) {
+                int pc = 0;
+#pragma unroll
+                for (int w = 0; w < D / 32; w++) pc += __builtin_popcount(~(qd.signs[lane][w] ^ token->signs[0][w]));
+                token->mq[lane] = (float)(2 * pc - D);
             }
-            __syncthreads();
+            if constexpr (RES) {
+                // (every key of the block is the token)
+                v4i_t acc = v4i_t{0, 0, 0, 0}, accl = v4i_t{0, 0, 0, 0};
+#pragma unroll
+                for (int m = 0; m < KB::kMfma; m++) {
+                    const int un = min(KB::unit(m, g4), D / 16 - 1);
+                    const v4i_t av = codes_i8(token->codes[0][2 * un], token->codes[0][2 * un + 1]);
+                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(*(const v4i_t*)&qd.bq[m][lane], av, acc, 0, 0, 0);
+                    if constexpr (3 * G > 16)
+                        accl = __builtin_amdgcn_mfma_i32_16x16x64_i8(*(const v4i_t*)&qd.bq_lo[m][lane], av, accl, 0, 0, 0);
+                }
+                if (lj == 0) {
+#pragma unroll
+                    for (int h = 0; h < 2; h++)
+                        if (2 * g4 + h < G) {
+                            token->dot[2 * g4 + h] = acc[2 * h] + 256 * acc[2 * h + 1];
+                            if constexpr (3 * G > 16) token->dot_lo[2 * g4 + h] = accl[2 * h];
+                        }
+                    if constexpr (3 * G <= 16) {
+#pragma unroll
+                        for (int g = 0; g < G; g++)
+                            if (g4 == (2 * G + g) / 4) token->dot_lo[g] = acc[(2 * G + g) % 4];
+                    }
+                }
+            }
+            // (the attention arguments hold the cache planes read-only)
+            const int64_t at = kv_base + slot;
+#pragma unroll
+            for (int v = 0; v < 2; v++) {
+                const BinPlanes& bp = v ? a.vb : a.kb;
+                const ResPlanes& rp = v ? a.vr : a.kr;
+                if (lane < D / 32) ((uint32_t*)(bp.signs + at * SB))[lane] = token->signs[v][lane];
+                if (lane == 0) ((uint16_t*)bp.scales)[at] = token->scale[v];
+                if constexpr (RES) {
+                    if (lane < D / 8) ((uint32_t*)(rp.codes + at * CB))[lane] = token->codes[v][lane];
+                    if (lane == 0) ((uint16_t*)rp.scales)[at] = token->rscale[v];
+                }
+            }
         }
     }
 
@@ -927,11 +984,11 @@ void attn_mfma_kernel(AttnArgs a) {
     // query digits of a single head in scalar registers for the whole loop
     // (uniform operands of v_dot8) when codes are read per key, and the int8
     // MFMA B operands of the K residual dot (loop invariant)
-    int sdig[(G == 1 && RES && !LIN_K) ? CW : 1][4];
-    // (groups of four and more: read per tile, their registers are full)
-    constexpr bool BQ_LDS = KMF && ALLRES && G >= 4;
+    int sdig[(RES && !KMF) ? CW : 1][4];
+    // (groups of four and more, and appending: read per tile, the registers are full)
+    constexpr bool BQ_LDS = KMF && ALLRES && (G >= 4 || APP);
     v4i_t bq[KMF && !BQ_LDS ? KB::kMfma : 1];
-    if constexpr (G == 1 && RES && !LIN_K) {
+    if constexpr (RES && !KMF) {
 #pragma unroll
         for (int w = 0; w < CW; w++) {
             const int4 dg = qd.digits[0][w];
@@ -1038,14 +1095,14 @@ void attn_mfma_kernel(AttnArgs a) {
             __builtin_amdgcn_s_waitcnt((n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8));
             __builtin_amdgcn_sched_barrier(0);
         }
-        const float sk = h2f(r.sk), svv = h2f(r.svv);
+        const float sk = h2f(r.sk);
+        float svv = h2f(r.svv);
         float rsk = h2f(r.rsk), rsv = h2f(r.rsv);
         uint32_t kc[KR::kCodeWords];
         if constexpr (RES) {
 #pragma unroll
             for (int w = 0; w < KR::kCodeWords; w++) kc[w] = r.kc[w];
         }
-
         float xd[G];
         uint32_t selmask = 0;
 #pragma unroll
@@ -1061,7 +1118,20 @@ void attn_mfma_kernel(AttnArgs a) {
                 for (int w = 0; w < D / 32; w++) pc += __builtin_popcount(~(qd.signs[g][w] ^ r.ks.w[w]));
             }
             const float mq = (float)(2 * pc - D);
-            xd[g] = (qd.scale_q[g] * sk) * mq;  // (scale_q * scale_k) * (2pc - d)  (src/xnor_dot.cuh:30)
+            xd[g] = xnor_score(qd.scale_q[g], sk, mq);
+        }
+        // (APP) the token's score parts and scales in place of the slot's key
+        const bool has_token = APP && t0 == app_t0;
+        if constexpr (APP) {
+            if (has_token && opaque_int(lane) == a.app_slot - t0) {
+                svv = h2f(token->scale[1]);
+                if constexpr (RES) {
+                    rsk = h2f(token->rscale[0]);
+                    rsv = h2f(token->rscale[1]);
+                }
+#pragma unroll
+                for (int g = 0; g < G; g++) xd[g] = xnor_score(qd.scale_q[g], h2f(token->scale[0]), token->mq[g]);
+            }
         }
         // adaptive: the tile's compacted residual positions (as in gather):
         // nsel selected keys, the lane's key at position rpos
@@ -1077,7 +1147,7 @@ void attn_mfma_kernel(AttnArgs a) {
             if (a.selected != nullptr && valid) {
 #pragma unroll
                 for (int g = 0; g < G; g++)
-                    a.selected[(int64_t)(bhq0 + g) * a.S + s] = (selmask >> g) & 1u;
+                    a.selected[(int64_t)(bhq0 + g) * S + s] = (selmask >> g) & 1u;
             }
         }
 
@@ -1153,6 +1223,18 @@ void attn_mfma_kernel(AttnArgs a) {
                     for (int g = 0; g < (LO_COLS && G > 1 ? G : 1); g++) rdlo[(16 * kb + lj) * G + g] = acc[kb][g];
                 }
             }
+            if constexpr (APP) {
+                // (APP) the token's dots over the slot's, after them
+                if (has_token) {
+                    const int rel = a.app_slot - t0, g = opaque_int(lane);
+                    if (g < G) {
+                        const int v = token->dot[g], vl = token->dot_lo[g];
+                        const bool joined = prec && (G == 1 || !LO_COLS);   // (one float, as above)
+                        rdl[rel * G + g] = joined ? __builtin_bit_cast(int, (float)v + (float)vl * (1.0f / 256.0f)) : v;
+                        if (G > 1 && LO_COLS) rdlo[rel * G + g] = vl;
+                    }
+                }
+            }
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -1174,124 +1256,26 @@ void attn_mfma_kernel(AttnArgs a) {
                     racc[g] = __builtin_bit_cast(int, (float)racc[g] + (float)rdlo[rpos * G + g] * (1.0f / 256.0f));
             }
           }
-        } else if constexpr (LIN_K) {
-            // round i: this lane holds 32 dims (quarter) of key i*(64/Q) + l/Q;
-            // partial dots are summed over the Q lanes of the row, and the lane
-            // whose own key it is keeps the total
-            int z;
-            asm volatile("v_mov_b32 %0, 0" : "=v"(z));  // keeps digit reads per tile (not hoisted)
-#pragma unroll
-            for (int i = 0; i < Q; i++) {
-#pragma unroll
-                for (int g = 0; g < G; g++) {
-                    int s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const int4 dg = qd.digits[g][4 * quarter + j + z];
-                        const int x = (int)kc[4 * i + j];
-                        s0 = __builtin_amdgcn_sdot8(dg.x, x, s0, false);
-                        s1 = __builtin_amdgcn_sdot8(dg.y, x, s1, false);
-                        s2 = __builtin_amdgcn_sdot8(dg.z, x, s2, false);
-                        s3 = __builtin_amdgcn_sdot8(dg.w, x, s3, false);
-                    }
-                    int tot = row_group_sum<Q>(s0 + 16 * s1 + 256 * s2 + 4096 * s3);
-                    if (G > 1 && prec) {
-                        // digits 0..1: the dot becomes tot + lo / 256 (float bits)
-                        int l0 = 0, l1 = 0;
-#pragma unroll
-                        for (int j = 0; j < 4; j++) {
-                            const int2 dl = qd.digits_lo[g][4 * quarter + j + z];
-                            const int x = (int)kc[4 * i + j];
-                            l0 = __builtin_amdgcn_sdot8(dl.x, x, l0, false);
-                            l1 = __builtin_amdgcn_sdot8(dl.y, x, l1, false);
-                        }
-                        const int totl = row_group_sum<Q>(l0 + 16 * l1);
-                        tot = __builtin_bit_cast(int, (float)tot + (float)totl * (1.0f / 256.0f));
-                    }
-                    racc[g] = quarter == i ? tot : racc[g];
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            if (G == 1 && prec) {
-                // (a single head: a separate pass keeps the register peak of
-                // the main loop) digits 0..1: the dot becomes racc + lo / 256
-#pragma unroll
-                for (int i = 0; i < Q; i++) {
-#pragma unroll
-                    for (int g = 0; g < G; g++) {
-                        int l0 = 0, l1 = 0;
-#pragma unroll
-                        for (int j = 0; j < 4; j++) {
-                            const int2 dl = qd.digits_lo[g][4 * quarter + j + z];
-                            const int x = (int)kc[4 * i + j];
-                            l0 = __builtin_amdgcn_sdot8(dl.x, x, l0, false);
-                            l1 = __builtin_amdgcn_sdot8(dl.y, x, l1, false);
-                        }
-                        const int totl = row_group_sum<Q>(l0 + 16 * l1);
-                        if (quarter == i)
-                            racc[g] = __builtin_bit_cast(int, (float)racc[g] + (float)totl * (1.0f / 256.0f));
-                    }
-                }
-            }
-        } else if constexpr (G == 1 && RES && !LIN_K) {
-            {
-                int s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-#pragma unroll
-                for (int w = 0; w < CW; w++) {
-                    s0 = __builtin_amdgcn_sdot8(sdig[w][0], (int)kc[w], s0, false);
-                    s1 = __builtin_amdgcn_sdot8(sdig[w][1], (int)kc[w], s1, false);
-                    s2 = __builtin_amdgcn_sdot8(sdig[w][2], (int)kc[w], s2, false);
-                    s3 = __builtin_amdgcn_sdot8(sdig[w][3], (int)kc[w], s3, false);
-                }
-                racc[0] = s0 + 16 * s1 + 256 * s2 + 4096 * s3;
-                if (prec) {
-                    int l0 = 0, l1 = 0;
-#pragma unroll
-                    for (int w = 0; w < CW; w++) {
-                        const int2 dl = qd.digits_lo[0][w];
-                        l0 = __builtin_amdgcn_sdot8(dl.x, (int)kc[w], l0, false);
-                        l1 = __builtin_amdgcn_sdot8(dl.y, (int)kc[w], l1, false);
-                    }
-                    racc[0] = __builtin_bit_cast(int, (float)racc[0] + (float)(l0 + 16 * l1) * (1.0f / 256.0f));
-                }
-            }
         } else if constexpr (RES) {
-            bool any_res = ALLRES;
-            if constexpr (MODE == MODE_ADAPTIVE) any_res = selmask != 0u;
-            if (any_res) {
-                int sa[G][4];
+            // (adaptive single heads: the lane's own key)
+            int s0 = 0, s1 = 0, s2 = 0, s3 = 0;
 #pragma unroll
-                for (int g = 0; g < G; g++) sa[g][0] = sa[g][1] = sa[g][2] = sa[g][3] = 0;
-                int z;
-                asm volatile("v_mov_b32 %0, 0" : "=v"(z));
+            for (int w = 0; w < CW; w++) {
+                s0 = __builtin_amdgcn_sdot8(sdig[w][0], (int)kc[w], s0, false);
+                s1 = __builtin_amdgcn_sdot8(sdig[w][1], (int)kc[w], s1, false);
+                s2 = __builtin_amdgcn_sdot8(sdig[w][2], (int)kc[w], s2, false);
+                s3 = __builtin_amdgcn_sdot8(sdig[w][3], (int)kc[w], s3, false);
+            }
+            racc[0] = s0 + 16 * s1 + 256 * s2 + 4096 * s3;
+            if (prec) {
+                int l0 = 0, l1 = 0;
 #pragma unroll
                 for (int w = 0; w < CW; w++) {
-#pragma unroll
-                    for (int g = 0; g < G; g++) {
-                        const int4 dg = qd.digits[g][w + z];
-                        sa[g][0] = __builtin_amdgcn_sdot8(dg.x, (int)kc[w], sa[g][0], false);
-                        sa[g][1] = __builtin_amdgcn_sdot8(dg.y, (int)kc[w], sa[g][1], false);
-                        sa[g][2] = __builtin_amdgcn_sdot8(dg.z, (int)kc[w], sa[g][2], false);
-                        sa[g][3] = __builtin_amdgcn_sdot8(dg.w, (int)kc[w], sa[g][3], false);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
+                    const int2 dl = qd.digits_lo[0][w];
+                    l0 = __builtin_amdgcn_sdot8(dl.x, (int)kc[w], l0, false);
+                    l1 = __builtin_amdgcn_sdot8(dl.y, (int)kc[w], l1, false);
                 }
-#pragma unroll
-                for (int g = 0; g < G; g++)
-                    racc[g] = sa[g][0] + 16 * sa[g][1] + 256 * sa[g][2] + 4096 * sa[g][3];
-                if (prec) {
-#pragma unroll
-                    for (int g = 0; g < G; g++) {
-                        int l0 = 0, l1 = 0;
-#pragma unroll
-                        for (int w = 0; w < CW; w++) {
-                            const int2 dl = qd.digits_lo[g][w + z];
-                            l0 = __builtin_amdgcn_sdot8(dl.x, (int)kc[w], l0, false);
-                            l1 = __builtin_amdgcn_sdot8(dl.y, (int)kc[w], l1, false);
-                        }
-                        racc[g] = __builtin_bit_cast(int, (float)racc[g] + (float)(l0 + 16 * l1) * (1.0f / 256.0f));
-                    }
-                }
+                racc[0] = __builtin_bit_cast(int, (float)racc[0] + (float)(l0 + 16 * l1) * (1.0f / 256.0f));
             }
         }
         float sc[G];
@@ -1305,7 +1289,7 @@ void attn_mfma_kernel(AttnArgs a) {
             // power of two; in a precise tile they are float bits already)
             const float rd = prec ? __builtin_bit_cast(float, racc[g]) : (float)racc[g];
             if (RES && use_res)
-                score = score + rd * (qd.dq[g] * (rsk * (KMF ? 1.0f / 112.0f : 1.0f / 7.0f)));
+                score = fmaf(rd, qd.dq[g] * (rsk * (KMF ? 1.0f / 112.0f : 1.0f / 7.0f)), score);
             sc[g] = valid ? score * isd2 : -INFINITY;
         }
 
@@ -1457,6 +1441,17 @@ void attn_mfma_kernel(AttnArgs a) {
             __builtin_amdgcn_s_waitcnt(0);
         }
         // (adaptive mode: the compiler waits for this staging buffer's loads)
+        if constexpr (APP) {
+            if (has_token) {   // the token's V row over the slot's
+                const int rel = a.app_slot - t0, ln = opaque_int(lane);
+                if (ln < SB / 4) ((uint32_t*)(st_signs + WL::kSignStride * rel))[ln] = token->signs[1][ln];
+                if constexpr (RES) {
+                    const int sw = Q_POW2 ? ((rel * CB) >> 8) & (Q - 1) : 0;
+                    if (ln < CB / 4)
+                        ((uint32_t*)(st_codes + CB * rel + 16 * ((ln >> 2) ^ sw)))[ln & 3] = token->codes[1][ln];
+                }
+            }
+        }
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the weight stores above
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -1817,7 +1812,7 @@ template <int D>
 bool launch_wide(int mode, int G, const AttnArgs& a, dim3 grid, hipStream_t st, int nw) {
     if constexpr (D == 64 || D == 128 || D == 256) {
         if (mode == MODE_BINARY && G == 1 && nw == 8) {
-            hipLaunchKernelGGL((attn_mfma_kernel<D, 1, MODE_BINARY, 8>), grid, dim3(8 * 64), 0, st, a);
+            hipLaunchKernelGGL((attn_mfma_kernel<D, 1, MODE_BINARY, 8>), grid, dim3(8 * 64), 0, st, BC_MFMA_ARGS(a, 1));
             return true;
         }
     }
@@ -1826,14 +1821,23 @@ bool launch_wide(int mode, int G, const AttnArgs& a, dim3 grid, hipStream_t st, 
 
 template <int D, int G>
 void launch_dg(int mode, const AttnArgs& a, dim3 grid, hipStream_t st) {
+    if constexpr (bc::append_dim(D)) {
+        if (a.app_k != nullptr) {
+            if (mode == MODE_BINARY)
+                hipLaunchKernelGGL((attn_mfma_kernel<D, G, MODE_BINARY, 4, true>), grid, dim3(256), 0, st, BC_MFMA_ARGS(a, G));
+            else
+                hipLaunchKernelGGL((attn_mfma_kernel<D, G, MODE_COMP, 4, true>), grid, dim3(256), 0, st, BC_MFMA_ARGS(a, G));
+            return;
+        }
+    }
     if (mode == MODE_BINARY)
-        hipLaunchKernelGGL((attn_mfma_kernel<D, G, MODE_BINARY>), grid, dim3(256), 0, st, a);
+        hipLaunchKernelGGL((attn_mfma_kernel<D, G, MODE_BINARY>), grid, dim3(256), 0, st, BC_MFMA_ARGS(a, G));
     else if (mode == MODE_COMP)
-        hipLaunchKernelGGL((attn_mfma_kernel<D, G, MODE_COMP>), grid, dim3(256), 0, st, a);
+        hipLaunchKernelGGL((attn_mfma_kernel<D, G, MODE_COMP>), grid, dim3(256), 0, st, BC_MFMA_ARGS(a, G));
     else if (mode == MODE_MIXED)
-        hipLaunchKernelGGL((attn_mfma_kernel<D, G, MODE_MIXED>), grid, dim3(256), 0, st, a);
+        hipLaunchKernelGGL((attn_mfma_kernel<D, G, MODE_MIXED>), grid, dim3(256), 0, st, BC_MFMA_ARGS(a, G));
     else
-        hipLaunchKernelGGL((attn_mfma_kernel<D, G, MODE_ADAPTIVE>), grid, dim3(256), 0, st, a);
+        hipLaunchKernelGGL((attn_mfma_kernel<D, G, MODE_ADAPTIVE>), grid, dim3(256), 0, st, BC_MFMA_ARGS(a, G));
 }
 
 template <int D, int G>
@@ -1857,6 +1861,8 @@ namespace bc {
 
 template <int D>
 bool mfma_launch(int mode, int G, const AttnArgs& a, dim3 grid, hipStream_t st, int nw) {
+    if ((a.Hq / a.Hkv) / G > kMaxHeadGroups) return false;
+    if (a.app_k != nullptr && (!append_dim(D) || mode == MODE_ADAPTIVE || mode == MODE_MIXED)) return false;
     if (nw != 4) return launch_wide<D>(mode, G, a, grid, st, nw);
     switch (G) {
         case 8: launch_dg<D, 8>(mode, a, grid, st); break;

@@ -139,7 +139,7 @@ def test_config_c4_full_size():
     (1, 16, 1, 128, 200, 150, 60, True),     # group 16: two query-head groups, two-launch path
     (2, 4, 2, 64, 130, 64, 80, False),       # binary caches, d = 64, wraps
     (1, 4, 4, 256, 96, 0, 120, True),        # d = 256, from empty, wraps
-    (1, 4, 2, 96, 64, 30, 50, True),         # d = 96: VALU kernels, two-launch path, wraps
+    (1, 4, 2, 96, 64, 30, 50, True),         # d = 96: two-launch path, wraps
 ])
 def test_append_attend_equals_append_then_attend(B, Hq, Hkv, d, max_seq, prefill, steps, comp):
     """BitCache.append_attend (one launch: the workgroup holding the ring slot
@@ -169,6 +169,35 @@ def test_append_attend_equals_append_then_attend(B, Hq, Hkv, d, max_seq, prefill
     if comp:
         pairs += [(a._k_res, b._k_res), (a._v_res, b._v_res)]
     for x, y in pairs:
+        assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("G", [1, 2, 4, 8])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_append_attend_on_precise_tiles(G, d):
+    """As above at unit variance (the residual dots of every tile take the
+    24-bit fixed point, the appended token's among them) for every head group:
+    the slot in the last tile of a 600-slot ring (its wave's second), then in
+    the first one, the token ten times larger than the keys around it, then
+    ten times smaller."""
+    from bitcache_amd import BitCache
+    say(f"case append_attend precise G={G} d={d}")
+    B, Hkv, max_seq, steps = 1, 2, 600, 30
+    g = torch.Generator(device="cuda")
+    g.manual_seed(100 * G + d)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda").half()
+    a = BitCache(B, Hkv * G, d, max_seq, n_kv_heads=Hkv)
+    b = BitCache(B, Hkv * G, d, max_seq, n_kv_heads=Hkv)
+    k0, v0 = rnd(B, Hkv, 585, d), rnd(B, Hkv, 585, d)
+    a.prefill(k0, v0)
+    b.prefill(k0, v0)
+    for t in range(steps):
+        scale = (1.0, 10.0, 0.1)[t % 3]
+        k, v, q = rnd(B, Hkv, d) * scale, rnd(B, Hkv, d) * scale, rnd(B, Hkv * G, d)
+        a.append(k, v)
+        want = a.attend(q)
+        assert torch.equal(b.append_attend(k, v, q), want), f"output differs at step {t}"
+    for x, y in ((a._k_bin, b._k_bin), (a._v_bin, b._v_bin), (a._k_res, b._k_res), (a._v_res, b._v_res)):
         assert torch.equal(x, y)
 
 
