@@ -116,12 +116,8 @@ class BitCache:
         assert K.dtype == torch.float16 and V.dtype == torch.float16
         assert K.is_contiguous() and V.is_contiguous()
         assert self._write_pos + S <= self.max_seq, "prefill would wrap the ring buffer"
-        for src, bin_, res in ((K, self._k_bin, self._k_res), (V, self._v_bin, self._v_res)):
-            if layout == "bhsd":
-                _C.encode_into_cache(src, bin_, res, B * H, S, d, self._write_pos, self.max_seq, True)
-            else:
-                _C.encode_into_cache_bshd(src, bin_, res, B, S, H, d, self._write_pos,
-                                          self.max_seq, True)
+        _C.encode_kv_into_cache(K, V, self._k_bin, self._k_res, self._v_bin, self._v_res, B, S, H, d,
+                                self._write_pos, self.max_seq, True, layout == "bshd")
         self._write_pos = (self._write_pos + S) % self.max_seq
         self._filled = min(self._filled + S, self.max_seq)
 

@@ -1,13 +1,10 @@
 // Encode kernels: fp16 vectors -> sign bits + fp16 mean-|x| scale (+ INT4 residual).
 //
-// One wave64 encodes one vector.  Lane l holds elements l + 64k (k < D/64),
-// which makes the sign words two (or one) wave ballots and lets the scale be
-// reduced in exactly the reference's fp32 order: the reference block has 128
-// threads, thread t summing |x_t| + |x_{t+128}| (src/binary_encode.cu:31-41),
-// followed by a shared-memory tree p[t] += p[t+s], s = 64..1 (:44-50).  Lane l
-// plays threads l and l+64; the s = 64 step is an in-lane add and the s = 32..1
-// steps are an xor butterfly whose lane-0 value follows the tree's association
-// exactly (fp32 addition is commutative).
+// A wave encodes several vectors at a time with a few lanes each (the two row
+// encoders below), in exactly the reference's fp32 order: the reference block
+// has 128 threads, thread t summing |x_t| + |x_{t+128}|
+// (src/binary_encode.cu:31-41), followed by a shared-memory tree
+// p[t] += p[t+s], s = 64..1 (:44-50).
 #include <math.h>
 
 #include <mutex>
@@ -50,6 +47,16 @@ __device__ __forceinline__ uint32_t fast_div(uint32_t n, const FastDiv& f) {
 // (b H + h) * row_stride + row_offset + s.  [rows, seq, d] sources are H = 1
 // (rows of S consecutive positions), [batch, seq, heads, d] sources H = heads,
 // one token per row S = 1.
+//
+// A wave iteration takes VPW vectors.  Linear order: consecutive
+// source vectors.  Blocked order (heads > 1 and at least VPW positions):
+// VPW consecutive positions of one head, 2^lg_t such iterations in turn for
+// each head of a block of positions, so that a wave's stores are whole runs of
+// a destination row (whole lines of the scale plane at 64 positions); the
+// source rows of one head (2 d bytes each, heads * 2 d apart) are whole lines
+// either way.  Linear order stored each of the wave's vectors in another row:
+// 4 x 16384 positions of 8 heads, d = 128: 48.7 us, blocked 36.5 us (39.0 us for the
+// same vectors as [rows, seq, d]).
 struct EncodeJob {
     const uint16_t* src;          // [n, D] fp16
     uint8_t* sign_plane;          // destination binary planes (ENC_RESIDUAL_ONLY: source)
@@ -59,6 +66,9 @@ struct EncodeJob {
     int64_t n;                    // vectors in this job (< 2^31)
     FastDiv H, S;
     int64_t row_stride, row_offset;
+    FastDiv blk;                  // blocked order: blocks of positions per batch
+    int lg_t;                     // ... and iterations per head and block
+    int64_t iters;                // wave iterations of the job
 };
 
 __device__ __forceinline__ int64_t dest_index(const EncodeJob& J, int64_t v) {
@@ -68,105 +78,6 @@ __device__ __forceinline__ int64_t dest_index(const EncodeJob& J, int64_t v) {
     const uint32_t b = fast_div(i, J.S);
     const uint32_t s = i - b * J.S.d;
     return (int64_t)(b * J.H.d + h) * J.row_stride + J.row_offset + s;
-}
-
-template <int D, int MODE>
-__global__ __launch_bounds__(256) void encode_kernel(EncodeJob j0, EncodeJob j1) {
-    constexpr int K = (D + 63) / 64;  // elements per lane
-    const int lane = threadIdx.x & 63;
-    const int64_t total = j0.n + j1.n;
-    const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x / 64);
-    for (int64_t gv = (int64_t)blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6); gv < total;
-         gv += nwaves) {
-        const bool second = gv >= j0.n;
-        const EncodeJob& J = second ? j1 : j0;
-        const int64_t v = second ? gv - j0.n : gv;
-        const int64_t dv = dest_index(J, v);
-
-        float x[K];
-        bool active[K];
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            const int e = lane + 64 * k;
-            active[k] = e < D;
-            x[k] = active[k] ? h2f(J.src[v * D + e]) : 0.0f;
-        }
-
-        float scale_for_residual;
-        uint64_t bits[K];
-        if constexpr (MODE == ENC_RESIDUAL_ONLY) {
-            const uint32_t* sp = (const uint32_t*)(J.sign_plane + dv * (D / 8));
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                const uint64_t lo = sp[2 * k];
-                const uint64_t hi = (2 * k + 1 < D / 32) ? sp[2 * k + 1] : 0u;
-                bits[k] = lo | (hi << 32);
-            }
-            scale_for_residual = h2f(J.scale_plane[dv]);
-        } else {
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                // x >= 0.0f: +-0 -> 1, NaN -> 0 (src/binary_encode.cu:36)
-                bits[k] = __ballot(active[k] && x[k] >= 0.0f);
-            }
-            // tree-order abs sum (see file comment).  Lane l is thread l (elements
-            // l, l+128) and thread l+64 (elements l+64, l+192); absent elements
-            // are 0 and adding them is exact.
-            float pA = 0.0f + fabsf(x[0]);
-            if constexpr (K > 2) pA = pA + fabsf(x[2]);
-            float pB = 0.0f;
-            if constexpr (K > 1) pB = pB + fabsf(x[1]);
-            if constexpr (K > 3) pB = pB + fabsf(x[3]);
-            float p = pA + pB;
-#pragma unroll
-            for (int s = 32; s > 0; s >>= 1) p = p + __shfl_xor(p, s, 64);
-            const float total_abs =
-                __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, p)));
-            const float mean = total_abs / (float)D;
-            if (lane == 0) J.scale_plane[dv] = f2h(mean);
-            // sign words: D/32 little-endian uint32 words per vector
-            uint32_t* sp = (uint32_t*)(J.sign_plane + dv * (D / 8));
-            if (lane < D / 32) {
-                uint64_t w = bits[0];
-#pragma unroll
-                for (int k = 1; k < K; k++) w = ((lane >> 1) == k) ? bits[k] : w;
-                sp[lane] = (lane & 1) ? (uint32_t)(w >> 32) : (uint32_t)w;
-            }
-            if constexpr (MODE == ENC_FUSED_FP16) scale_for_residual = h2f(f2h(mean));
-            else scale_for_residual = mean;
-        }
-
-        if constexpr (MODE != ENC_BINARY) {
-            if (J.code_plane == nullptr) continue;
-            const float s = scale_for_residual;
-            float r[K];
-            float m = 0.0f;
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                const bool b = (bits[k] >> lane) & 1ull;
-                r[k] = x[k] - (b ? s : -s);
-                if (active[k]) m = fmaxf(m, fabsf(r[k]));
-            }
-            // fmaxf ignores NaN and is order independent: a butterfly gives the
-            // reference's absmax (src/residual.cu:30-53) in every lane.
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-            const float absmax = m;
-            const float inv = absmax > 0.0f ? 7.0f / absmax : 0.0f;
-            if (lane == 0) J.rscale_plane[dv] = f2h(absmax);
-            uint8_t* cp = J.code_plane + dv * (D / 2);
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                // element e = lane + 64k; element 2j -> low nibble of byte j
-                uint32_t c = (uint32_t)quant7(r[k] * inv) & 0xFu;
-                uint32_t byte = c | (__shfl_xor(c, 1, 64) << 4);          // valid on even lanes
-                uint32_t half = byte | (__shfl_xor(byte, 2, 64) << 8);     // lanes % 4 == 0
-                uint32_t word = half | (__shfl_xor(half, 4, 64) << 16);    // lanes % 8 == 0
-                const int e = lane + 64 * k;
-                if ((lane & 7) == 0 && e < D) ((uint32_t*)cp)[e >> 3] = word;
-            }
-        }
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -197,6 +108,18 @@ __global__ __launch_bounds__(256) void encode_kernel(EncodeJob j0, EncodeJob j1)
 // (fma(a, 1, b) is the single-rounded sum, equal to the fp32 add of the
 // exactly converted halves); `one` is an fp16 1.0 the compiler cannot fold,
 // so it keeps the fma rather than rewriting it to convert + add.
+// Eight codes of the fast path (|y| < 7.5) as a dword.
+__device__ __forceinline__ uint32_t pack_codes(const float* y) {
+    uint32_t c[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) c[k] = __builtin_bit_cast(uint32_t, y[k] + 12582920.0f);
+    const uint32_t p0 = (c[1] << 4) | c[0], p1 = (c[3] << 4) | c[2];
+    const uint32_t p2 = (c[5] << 4) | c[4], p3 = (c[7] << 4) | c[6];
+    const uint32_t t0 = __builtin_amdgcn_perm(p1, p0, 0x0C0C0400u);   // p0.b0, p1.b0
+    const uint32_t t1 = __builtin_amdgcn_perm(p3, p2, 0x0C0C0400u);   // p2.b0, p3.b0
+    return __builtin_amdgcn_perm(t1, t0, 0x05040100u) ^ 0x88888888u;
+}
+
 template <int D, int MODE>
 __device__ __forceinline__ void encode_two_slices(const bc_v4u ra, const bc_v4u rb, int j, bool live,
                                                   const EncodeDst& dst, int64_t dv, _Float16 one) {
@@ -343,18 +266,8 @@ __device__ __forceinline__ void encode_two_slices(const bc_v4u ra, const bc_v4u 
         }
         uint32_t word_a, word_b;
         if (__ballot(!finite) == 0ull) {
-            auto pack = [](const float* y) -> uint32_t {
-                uint32_t c[8];
-#pragma unroll
-                for (int k = 0; k < 8; k++) c[k] = __builtin_bit_cast(uint32_t, y[k] + 12582920.0f);
-                const uint32_t p0 = (c[1] << 4) | c[0], p1 = (c[3] << 4) | c[2];
-                const uint32_t p2 = (c[5] << 4) | c[4], p3 = (c[7] << 4) | c[6];
-                const uint32_t t0 = __builtin_amdgcn_perm(p1, p0, 0x0C0C0400u);   // p0.b0, p1.b0
-                const uint32_t t1 = __builtin_amdgcn_perm(p3, p2, 0x0C0C0400u);   // p2.b0, p3.b0
-                return __builtin_amdgcn_perm(t1, t0, 0x05040100u) ^ 0x88888888u;
-            };
-            word_a = pack(y_a);
-            word_b = pack(y_b);
+            word_a = pack_codes(y_a);
+            word_b = pack_codes(y_b);
         } else {
             word_a = word_b = 0;
 #pragma unroll
@@ -372,14 +285,146 @@ __device__ __forceinline__ void encode_two_slices(const bc_v4u ra, const bc_v4u 
     }
 }
 
-// Row-parallel encoder for d in {64, 128, 256}: 64/P vectors per wave
-// iteration (encode_two_slices), coalesced loads and stores, all reductions
-// on DPP / swizzle lane moves.  Same results as encode_kernel.
+// Column encoder for the other multiples of 32 (32, 96, 160, 192, 224): eight
+// lanes per vector, lane j holding elements 64k + 8j .. 64k + 8j + 7 of every
+// 64-element block k (the last block of d % 64 == 32 is half: lanes 4..7 hold
+// zeros there, whose terms are exact +0.0).  The reference's thread t sums
+// |x_t| + |x_{t+128}|, its s = 64 step pairs t with t + 64: in-lane adds over
+// the blocks; s = 32, 16, 8 pair lane j with j + 4, 2, 1 and s = 4, 2, 1 are
+// in-lane: the reference tree's association exactly.  One wave per vector (the
+// kernel that ran these head dims, shuffles and 2-byte loads) took 4.7 times
+// as long: 524288 vectors of d = 96 139.7 -> 42.1 us (3.2 TB/s).
 template <int D, int MODE>
+__device__ __forceinline__ void encode_columns(const bc_v4u (&raw)[(D + 63) / 64], int j, bool live,
+                                               const EncodeDst& dst, int64_t dv) {
+    constexpr int K = (D + 63) / 64;
+    constexpr bool HALF = D % 64 != 0;
+    float x[K][8];
+    bool pos[K][8];   // x >= 0: +-0 -> 1, NaN -> 0 (src/binary_encode.cu:36)
+    uint32_t bytes[K];
+#pragma unroll
+    for (int k = 0; k < K; k++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) x[k][e] = h2f((uint16_t)(raw[k][e >> 1] >> (16 * (e & 1))));
+    // (a lane past the last block's elements)
+    const bool pad = HALF && j >= 4;
+    float s;
+    if constexpr (MODE == ENC_RESIDUAL_ONLY) {
+        const uint8_t* sp = dst.sign_plane + dv * (D / 8);
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            bytes[k] = (k == K - 1 && pad) ? 0u : sp[8 * k + j];
+#pragma unroll
+            for (int e = 0; e < 8; e++) pos[k][e] = (bytes[k] >> e) & 1u;
+        }
+        s = h2f(dst.scale_plane[dv]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            bytes[k] = 0;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                pos[k][e] = x[k][e] >= 0.0f;
+                bytes[k] |= (pos[k][e] ? 1u : 0u) << e;
+            }
+        }
+        float p[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            float pa = fabsf(x[0][e]), pb = 0.0f;
+            if constexpr (K > 2) pa = pa + fabsf(x[2][e]);
+            if constexpr (K > 1) pb = fabsf(x[1][e]);
+            if constexpr (K > 3) pb = pb + fabsf(x[3][e]);
+            p[e] = pa + pb;                                                  // s = 64
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) p[e] = p[e] + dpp_f<0x104>(p[e]);       // s = 32
+#pragma unroll
+        for (int e = 0; e < 8; e++) p[e] = p[e] + dpp_f<0x102>(p[e]);       // s = 16
+#pragma unroll
+        for (int e = 0; e < 8; e++) p[e] = p[e] + dpp_f<0x101>(p[e]);       // s = 8
+#pragma unroll
+        for (int e = 0; e < 4; e++) p[e] = p[e] + p[e + 4];                  // s = 4
+        p[0] = p[0] + p[2];
+        p[1] = p[1] + p[3];                                                   // s = 2
+        p[0] = p[0] + p[1];                                                   // s = 1
+        const float mean = swz_f<0x18>(p[0]) / (float)D;   // (lane 0 of the eight)
+        if constexpr (MODE == ENC_FUSED_FP16) s = h2f(f2h(mean));
+        else s = mean;
+        // sign bytes of four lanes -> one dword
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const uint32_t w = bytes[k] | (dpp_u<0x101>(bytes[k]) << 8) | (dpp_u<0x102>(bytes[k]) << 16) |
+                               (dpp_u<0x103>(bytes[k]) << 24);
+            if (live && (j & 3) == 0 && !(k == K - 1 && pad))
+                *(uint32_t*)(dst.sign_plane + dv * (D / 8) + 8 * k + j) = w;
+        }
+        if (live && j == 0) dst.scale_plane[dv] = f2h(mean);
+    }
+    if constexpr (MODE != ENC_BINARY) {
+        if (dst.code_plane == nullptr) return;
+        float m = 0.0f;
+#pragma unroll
+        for (int k = 0; k < K; k++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                x[k][e] = x[k][e] - (pos[k][e] ? s : -s);   // the residual
+                // fmaxf ignores NaN and is order independent (src/residual.cu:30-53)
+                if (!(k == K - 1 && pad)) m = fmaxf(m, fabsf(x[k][e]));
+            }
+        // (non-negative and never NaN: the integer order is the float order)
+        uint32_t mb = __builtin_bit_cast(uint32_t, m);
+        mb = max(mb, dpp_u<0x141>(mb));   // half mirror
+        mb = max(mb, dpp_u<0x4E>(mb));
+        mb = max(mb, dpp_u<0xB1>(mb));
+        const float absmax = __builtin_bit_cast(float, mb);
+        const float inv = absmax > 0.0f ? 7.0f / absmax : 0.0f;
+        // (as in encode_two_slices: the mean is finite only if each element is;
+        // against a stored scale, 0 * residual summed is 0 only then)
+        float probe = s;
+        if constexpr (MODE == ENC_RESIDUAL_ONLY) {
+            probe = 0.0f;
+#pragma unroll
+            for (int k = 0; k < K; k++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) probe = fmaf(x[k][e], 0.0f, probe);
+        }
+        const bool exact = __ballot(!__builtin_isfinite(probe) || !__builtin_isfinite(inv)) != 0ull;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            float y[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) y[e] = x[k][e] * inv;
+            uint32_t word = 0;
+            if (!exact) {
+                word = pack_codes(y);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++) word |= ((uint32_t)quant7(y[e]) & 0xFu) << (4 * e);
+            }
+            if (live && !(k == K - 1 && pad)) ((uint32_t*)(dst.code_plane + dv * (D / 2)))[8 * k + j] = word;
+        }
+        if (live && j == 0) dst.rscale_plane[dv] = f2h(absmax);
+    }
+}
+
+// The two row encoders behind one face: lanes per vector, the slices a lane
+// loads, and the encode.
+__host__ __device__ constexpr bool two_slices(int D) { return D == 64 || D == 128 || D == 256; }
+__host__ __device__ constexpr int row_lanes(int D) { return two_slices(D) ? D / 16 : 8; }
+__host__ __device__ constexpr int row_slices(int D) { return two_slices(D) ? 2 : (D + 63) / 64; }
+
+// Row-parallel encoder: 64 / row_lanes(D) vectors per wave iteration,
+// coalesced loads and stores, all reductions on DPP / swizzle lane moves.
+// BLK: the jobs' blocked order (EncodeJob), else the linear one.
+template <int D, int MODE, bool BLK>
 __global__ __launch_bounds__(256) void encode_rows_kernel(EncodeJob j0, EncodeJob j1, int lg_run) {
-    static_assert(D == 64 || D == 128 || D == 256, "row encoder: d in {64, 128, 256}");
-    constexpr int L = D / 16;       // lanes per vector
-    constexpr int VPW = 64 / L;     // vectors per wave
+    constexpr int L = row_lanes(D);   // lanes per vector
+    constexpr int VPW = 64 / L;       // vectors per wave
+    constexpr int NS = row_slices(D);
+    // an iteration's index steps by 1 in blocked order, by its vectors in
+    // linear order (the index of its first one)
+    constexpr int UNIT = BLK ? 1 : VPW;
     const int lane = threadIdx.x & 63;
     const int sub = lane / L, j = lane % L;
     // (readfirstlane: the wave index is uniform, so the loop below runs on
@@ -387,8 +432,8 @@ __global__ __launch_bounds__(256) void encode_rows_kernel(EncodeJob j0, EncodeJo
     const int64_t wave_id = (int64_t)blockIdx.x * (blockDim.x >> 6) +
                             __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x >> 6);
-    // the next iteration's slice is loaded before this one is encoded, so
-    // each wave keeps two 16-byte loads per lane in flight
+    // the next iteration's slices are loaded before this one is encoded, so
+    // each wave keeps NS 16-byte loads per lane in flight
 #pragma unroll 1
     for (int jb = 0; jb < 2; jb++) {
         const EncodeJob& J = jb ? j1 : j0;
@@ -399,82 +444,111 @@ __global__ __launch_bounds__(256) void encode_rows_kernel(EncodeJob j0, EncodeJo
             wid += nwaves / 2;
             if (wid >= nwaves) wid -= nwaves;
         }
-        // (jobs hold fewer than 2^31 vectors: 32-bit vector indices)
-        auto vec_of = [&](int64_t b) -> int64_t {
-            return (int64_t)min((uint32_t)b + (uint32_t)sub, (uint32_t)J.n - 1u);
+        // blocked order: it = ((batch * blocks + block) * H + h) * 2^lg_t + t
+        struct Pos {
+            uint32_t b, h, s0;   // the iteration's batch, head and first position
         };
-        // destination of this lane's vector b + sub: when the wave's VPW
-        // vectors sit in one row (H = 1: consecutive positions) or in one
-        // (batch, position) (consecutive heads), one scalar index computation
-        // for the wave, else per lane
-        auto dest_for = [&](int64_t b) -> int64_t {
-            const uint32_t u = (uint32_t)b;
+        auto pos_of = [&](int64_t it) -> Pos {
+            const uint32_t t = (uint32_t)it & ((1u << J.lg_t) - 1u), u = (uint32_t)(it >> J.lg_t);
+            const uint32_t i = fast_div(u, J.H), h = u - i * J.H.d;
+            const uint32_t b = fast_div(i, J.blk), blk = i - b * J.blk.d;
+            return Pos{b, h, ((blk << J.lg_t) + t) * VPW};
+        };
+        // this lane's source vector (clamped), whether it holds one, and its
+        // destination (jobs hold fewer than 2^31 vectors: 32-bit indices)
+        auto vec_of = [&](int64_t it) -> int64_t {
+            if constexpr (BLK) {
+                const Pos p = pos_of(it);
+                return ((int64_t)p.b * J.S.d + min(p.s0 + (uint32_t)sub, J.S.d - 1u)) * J.H.d + p.h;
+            }
+            return (int64_t)min((uint32_t)it + (uint32_t)sub, (uint32_t)J.n - 1u);
+        };
+        auto live_of = [&](int64_t it) -> bool {
+            if constexpr (BLK) return pos_of(it).s0 + (uint32_t)sub < J.S.d;
+            return it + sub < J.n;
+        };
+        // (linear order: when the wave's vectors sit in one row, H = 1:
+        // consecutive positions, or in one (batch, position): consecutive
+        // heads, one scalar index computation for the wave, else per lane)
+        auto dest_for = [&](int64_t it) -> int64_t {
+            if constexpr (BLK) {
+                const Pos p = pos_of(it);
+                return (int64_t)(p.b * J.H.d + p.h) * J.row_stride + J.row_offset + p.s0 + sub;
+            }
+            const uint32_t u = (uint32_t)it;
             const uint32_t i = fast_div(u, J.H);
             const uint32_t h = u - i * J.H.d;
             const uint32_t bb = fast_div(i, J.S);
             const uint32_t s = i - bb * J.S.d;
-            const bool run = b + VPW <= J.n && (J.H.d == 1 ? s + VPW <= J.S.d : h + VPW <= J.H.d);
+            const bool run = it + VPW <= J.n && (J.H.d == 1 ? s + VPW <= J.S.d : h + VPW <= J.H.d);
             if (run)
                 return (int64_t)(bb * J.H.d + h) * J.row_stride + J.row_offset + s +
                        (int64_t)sub * (J.H.d == 1 ? 1 : J.row_stride);
-            return dest_index(J, vec_of(b));
+            return dest_index(J, vec_of(it));
         };
         const EncodeDst dst{J.sign_plane, J.scale_plane, J.code_plane, J.rscale_plane};
-        // each wave encodes runs of 2^lg_run x VPW consecutive vectors (runs
-        // of 16 write the cache lines of the scale and sign planes whole from
-        // one wave, i.e. one L2, rather than in pieces from several XCDs;
-        // small jobs take runs of 1 to spread over the waves).  Iteration t of
-        // the wave starts at ((t >> lg) nwaves + wid) VPW 2^lg + (t mod 2^lg) VPW,
-        // stepped incrementally: +VPW inside a run, +jump to the next run.
+        // each wave takes runs of 2^lg_run consecutive iterations (runs of 16
+        // write the cache lines of the scale and sign planes whole from one
+        // wave, i.e. one L2, rather than in pieces from several XCDs; small
+        // jobs take runs of 1 to spread over the waves).  Iteration n of the
+        // wave is number ((n >> lg) nwaves + wid) 2^lg + (n mod 2^lg), stepped
+        // incrementally.
         const int run = 1 << lg_run;
-        const int64_t jump = (int64_t)VPW + (nwaves - 1) * ((int64_t)run * VPW);
-        auto step = [&](int64_t b, int& pos) -> int64_t {
+        const int64_t jump = UNIT + (nwaves - 1) * ((int64_t)run * UNIT);
+        const int64_t end = BLK ? J.iters : J.n;
+        auto step = [&](int64_t it, int& pos) -> int64_t {
             if (++pos == run) {
                 pos = 0;
-                return b + jump;
+                return it + jump;
             }
-            return b + VPW;
+            return it + UNIT;
         };
         // fp16 1.0 hidden from constant folding (see encode_two_slices)
         _Float16 one = (_Float16)1.0f;
         asm volatile("" : "+v"(one));
-        // slices A and B of this lane's vector (nontemporal: each wave's
-        // vectors are one contiguous run read once)
-        auto load = [&](int64_t b, bc_v4u& a, bc_v4u& bb) {
-            const bc_v4u* p = (const bc_v4u*)(J.src + vec_of(b) * D) + j;
-            a = __builtin_nontemporal_load(p);
-            bb = __builtin_nontemporal_load(p + D / 16);
+        // this lane's slices of its vector (nontemporal: read once)
+        auto load = [&](int64_t it, bc_v4u (&r)[NS]) {
+            const bc_v4u* p = (const bc_v4u*)(J.src + vec_of(it) * D) + j;
+#pragma unroll
+            for (int k = 0; k < NS; k++) {
+                if constexpr (two_slices(D)) {
+                    r[k] = __builtin_nontemporal_load(p + k * (D / 16));
+                } else {
+                    // (the half block's lanes past it read nothing)
+                    const bool in = D % 64 == 0 || k < NS - 1 || j < 4;
+                    const bc_v4u z = {0u, 0u, 0u, 0u};
+                    r[k] = in ? __builtin_nontemporal_load(p + k * 8) : z;
+                }
+            }
+        };
+        auto encode = [&](const bc_v4u (&r)[NS], int64_t it) {
+            if constexpr (two_slices(D)) encode_two_slices<D, MODE>(r[0], r[1], j, live_of(it), dst, dest_for(it), one);
+            else encode_columns<D, MODE>(r, j, live_of(it), dst, dest_for(it));
         };
         // two register sets used in turn (a copy between them would wait for
         // the load in flight); the prefetch is issued unconditionally (past
         // the last iteration it reloads the current slices) so that the wait
         // before each encode leaves it in flight
-        int64_t base = wid * ((int64_t)run * VPW);
-        if (base >= J.n) continue;
-        int pos = 0;   // (wave-uniform: base, pos and nb run on scalar registers)
-        bc_v4u ra, rb, qa, qb;
-        load(base, ra, rb);
+        int64_t it = wid * ((int64_t)run * UNIT);
+        if (it >= end) continue;
+        int pos = 0;   // (wave-uniform: it, pos and ni run on scalar registers)
+        bc_v4u r0[NS], r1[NS];
+        load(it, r0);
         for (;;) {
-            int64_t nb = step(base, pos);
-            bool more = nb < J.n;
-            load(more ? nb : base, qa, qb);
-            encode_two_slices<D, MODE>(ra, rb, j, base + sub < J.n, dst, dest_for(base), one);
+            int64_t ni = step(it, pos);
+            bool more = ni < end;
+            load(more ? ni : it, r1);
+            encode(r0, it);
             if (!more) break;
-            base = nb;
-            nb = step(base, pos);
-            more = nb < J.n;
-            load(more ? nb : base, ra, rb);
-            encode_two_slices<D, MODE>(qa, qb, j, base + sub < J.n, dst, dest_for(base), one);
+            it = ni;
+            ni = step(it, pos);
+            more = ni < end;
+            load(more ? ni : it, r0);
+            encode(r1, it);
             if (!more) break;
-            base = nb;
+            it = ni;
         }
     }
-}
-
-int grid_for(int64_t nvec) {
-    const int64_t want = (nvec + 3) / 4;
-    const int64_t cap = (int64_t)bc::device_cu_count() * 32;
-    return (int)(want < cap ? (want < 1 ? 1 : want) : cap);
 }
 
 // Blocks per CU of the row encoder: 3 (12 waves per CU) measured fastest for
@@ -486,59 +560,78 @@ constexpr int kEncodeBlocksPerCU = 3;
 // 256-thread blocks of `kernel` resident per CU (occupancy query, once per
 // kernel; at least 1)
 template <int MODE>
-int resident_blocks(int d, void (*kernel)(EncodeJob, EncodeJob, int)) {
+int resident_blocks(int d, bool blk, void (*kernel)(EncodeJob, EncodeJob, int)) {
     static std::mutex mu;
-    static int cached[3] = {0, 0, 0};
-    const int slot = d == 64 ? 0 : (d == 128 ? 1 : 2);
+    static int cached[2][9] = {};
+    const int slot = d / 32;
     std::lock_guard<std::mutex> lock(mu);
-    if (cached[slot] == 0) {
+    if (cached[blk][slot] == 0) {
         int n = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, 256, 0) != hipSuccess || n < 1) n = 1;
-        cached[slot] = n;
+        cached[blk][slot] = n;
     }
-    return cached[slot];
+    return cached[blk][slot];
+}
+
+// Wave iterations of a job of `vpw` vectors each.  Blocked order where a
+// [batch, seq, heads, d] row holds enough positions: blocks of up to 64, at
+// most an eighth of a row, so that the last block's padding stays small.
+void order_job(EncodeJob& j, int vpw, bool blk) {
+    if (j.n == 0) return;
+    if (!blk) {
+        j.iters = (j.n + vpw - 1) / vpw;
+        return;
+    }
+    while ((vpw << (j.lg_t + 1)) <= 64 && (uint32_t)(vpw << (j.lg_t + 1)) * 8 <= j.S.d) j.lg_t++;
+    const uint32_t per = (uint32_t)vpw << j.lg_t;
+    j.blk = make_fastdiv((j.S.d + per - 1) / per);
+    j.iters = (j.n / j.S.d) * j.blk.d << j.lg_t;   // (n / S = batches * heads)
 }
 
 template <int MODE>
-int launch_encode(int d, const EncodeJob& a, const EncodeJob& b, hipStream_t st) {
-    if (d == 64 || d == 128 || d == 256) {
-        // row encoder: 64/P vectors per wave, 4 waves per block, grid-stride
-        // over at most kEncodeBlocksPerCU blocks per CU, all resident at once
-        // (a grid of several rounds ends with a round at low occupancy)
-        auto kernel = d == 64 ? encode_rows_kernel<64, MODE>
-                              : (d == 128 ? encode_rows_kernel<128, MODE> : encode_rows_kernel<256, MODE>);
-        const int per_cu = resident_blocks<MODE>(d, kernel);
-        const int64_t cap =
-            (int64_t)bc::device_cu_count() * (per_cu < kEncodeBlocksPerCU ? per_cu : kEncodeBlocksPerCU);
-        // a grid of one iteration per wave if that fits, else the resident
-        // blocks with runs of up to 16 iterations (at most a quarter of each
-        // wave's, a power of two)
-        const int64_t vpw = 64 / (d / 16);
-        const int64_t one_pass = (a.n + b.n + 4 * vpw - 1) / (4 * vpw);
-        const int grid = (int)(one_pass < cap ? (one_pass < 1 ? 1 : one_pass) : cap);
-        const int64_t per_wave = (a.n + b.n + (int64_t)grid * 4 * vpw - 1) / ((int64_t)grid * 4 * vpw);
-        int lg_run = 0;
-        while (lg_run < 4 && (int64_t)(2 << lg_run) * 4 <= per_wave) lg_run++;
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, st, a, b, lg_run);
-        return bc::check_launch("encode");
-    }
-    if constexpr (MODE == ENC_TRAFFIC) {
-        return bc::set_error(BC_ERR_UNSUPPORTED, "traffic probe: head_dim %d unsupported", d);
-    } else {
-        const int grid = grid_for(a.n + b.n);
-        switch (d) {
-#define BC_CASE(DD)                                                                           \
-    case DD:                                                                                  \
-        hipLaunchKernelGGL((encode_kernel<DD, MODE>), dim3(grid), dim3(256), 0, st, a, b);     \
+int launch_encode(int d, EncodeJob a, EncodeJob b, hipStream_t st) {
+    // row encoder, 4 waves per block, grid-stride over at most
+    // kEncodeBlocksPerCU blocks per CU, all resident at once (a grid of
+    // several rounds ends with a round at low occupancy)
+    void (*kernel)(EncodeJob, EncodeJob, int) = nullptr;
+    int vpw = 0;
+    bool blk = false;
+    // (the jobs of a launch have one shape)
+#define BC_CASE(DD)                                                                                  \
+    case DD:                                                                                         \
+        vpw = 64 / row_lanes(DD);                                                                    \
+        blk = MODE != ENC_TRAFFIC && MODE != ENC_RESIDUAL_ONLY && a.H.d > 1 && a.S.d >= (uint32_t)vpw; \
+        kernel = blk ? encode_rows_kernel<DD, MODE, MODE != ENC_TRAFFIC && MODE != ENC_RESIDUAL_ONLY> \
+                     : encode_rows_kernel<DD, MODE, false>;                                          \
         break;
-            BC_CASE(32) BC_CASE(64) BC_CASE(96) BC_CASE(128) BC_CASE(160) BC_CASE(192) BC_CASE(224)
-            BC_CASE(256)
-#undef BC_CASE
-            default:
-                return bc::set_error(BC_ERR_UNSUPPORTED, "head_dim %d unsupported", d);
-        }
-        return bc::check_launch("encode");
+    switch (d) {
+        BC_CASE(64) BC_CASE(128) BC_CASE(256)
+        default: break;
     }
+    if constexpr (MODE != ENC_TRAFFIC) {
+        switch (d) {
+            BC_CASE(32) BC_CASE(96) BC_CASE(160) BC_CASE(192) BC_CASE(224)
+            default: break;
+        }
+    }
+#undef BC_CASE
+    if (kernel == nullptr) return bc::set_error(BC_ERR_UNSUPPORTED, "head_dim %d unsupported", d);
+    order_job(a, vpw, blk);
+    order_job(b, vpw, blk);
+    const int per_cu = resident_blocks<MODE>(d, blk, kernel);
+    const int64_t cap =
+        (int64_t)bc::device_cu_count() * (per_cu < kEncodeBlocksPerCU ? per_cu : kEncodeBlocksPerCU);
+    // a grid of one iteration per wave if that fits, else the resident
+    // blocks with runs of up to 16 iterations (at most a quarter of each
+    // wave's, a power of two)
+    const int64_t iters = a.iters + b.iters;
+    const int64_t one_pass = (iters + 3) / 4;
+    const int grid = (int)(one_pass < cap ? (one_pass < 1 ? 1 : one_pass) : cap);
+    const int64_t per_wave = (iters + (int64_t)grid * 4 - 1) / ((int64_t)grid * 4);
+    int lg_run = 0;
+    while (lg_run < 4 && (int64_t)(2 << lg_run) * 4 <= per_wave) lg_run++;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, st, a, b, lg_run);
+    return bc::check_launch("encode");
 }
 
 EncodeJob make_job(const void* src, void* bin, void* res, int64_t n, int64_t cap, int d,
@@ -667,9 +760,10 @@ extern "C" int bc_online_encode_kv(const void* k, const void* v, void* k_bin, vo
                          max_seq, stream);
 }
 
-static int encode_into_cache(const void* src, void* binary_cache, void* residual_cache,
-                             int64_t rows, int64_t heads, int seq, int head_dim, int start_pos,
-                             int max_seq, int scale_mode, void* stream) {
+// One source (v null) or a K and a V source of the same shape, in one launch.
+static int encode_into_cache(const void* k, const void* v, void* k_bin, void* k_res, void* v_bin,
+                             void* v_res, int64_t rows, int64_t heads, int seq, int head_dim,
+                             int start_pos, int max_seq, int scale_mode, void* stream) {
     BC_REQUIRE(bc::head_dim_ok(head_dim), BC_ERR_UNSUPPORTED,
                "head_dim must be a multiple of 32 in [32, 256], got %d", head_dim);
     BC_REQUIRE(rows >= 0 && heads > 0 && rows % heads == 0 && seq >= 0 && start_pos >= 0 &&
@@ -681,13 +775,13 @@ static int encode_into_cache(const void* src, void* binary_cache, void* residual
                "scale_mode must be 0 or 1");
     if (rows * seq == 0) return BC_OK;
     BC_REQUIRE(rows * seq <= INT32_MAX, BC_ERR_INVALID_ARGUMENT, "more than 2^31 - 1 vectors");
-    BC_REQUIRE(src && binary_cache, BC_ERR_INVALID_ARGUMENT, "null pointer");
+    BC_REQUIRE(k && k_bin && (!v || v_bin), BC_ERR_INVALID_ARGUMENT, "null pointer");
     const int64_t cap = rows * max_seq;
-    EncodeJob a = make_job(src, binary_cache, residual_cache, rows * seq, cap, head_dim, heads, seq,
-                           max_seq, start_pos);
+    EncodeJob a = make_job(k, k_bin, k_res, rows * seq, cap, head_dim, heads, seq, max_seq, start_pos);
     EncodeJob b{};
+    if (v) b = make_job(v, v_bin, v_res, rows * seq, cap, head_dim, heads, seq, max_seq, start_pos);
     hipStream_t st = (hipStream_t)stream;
-    if (!residual_cache) return launch_encode<ENC_BINARY>(head_dim, a, b, st);
+    if (!k_res) return launch_encode<ENC_BINARY>(head_dim, a, b, st);
     if (scale_mode == 0) return launch_encode<ENC_FUSED_FP16>(head_dim, a, b, st);
     return launch_encode<ENC_FUSED_FP32>(head_dim, a, b, st);
 }
@@ -695,14 +789,29 @@ static int encode_into_cache(const void* src, void* binary_cache, void* residual
 extern "C" int bc_encode_into_cache(const void* src, void* binary_cache, void* residual_cache,
                                     int64_t rows, int seq, int head_dim, int start_pos,
                                     int max_seq, int scale_mode, void* stream) {
-    return encode_into_cache(src, binary_cache, residual_cache, rows, 1, seq, head_dim, start_pos,
-                             max_seq, scale_mode, stream);
+    return encode_into_cache(src, nullptr, binary_cache, residual_cache, nullptr, nullptr, rows, 1, seq,
+                             head_dim, start_pos, max_seq, scale_mode, stream);
 }
 
 extern "C" int bc_encode_into_cache_bshd(const void* src, void* binary_cache, void* residual_cache,
                                          int batch, int seq, int n_heads, int head_dim,
                                          int start_pos, int max_seq, int scale_mode, void* stream) {
     BC_REQUIRE(batch >= 0 && n_heads > 0, BC_ERR_INVALID_ARGUMENT, "invalid batch / n_heads");
-    return encode_into_cache(src, binary_cache, residual_cache, (int64_t)batch * n_heads, n_heads,
-                             seq, head_dim, start_pos, max_seq, scale_mode, stream);
+    return encode_into_cache(src, nullptr, binary_cache, residual_cache, nullptr, nullptr,
+                             (int64_t)batch * n_heads, n_heads, seq, head_dim, start_pos, max_seq,
+                             scale_mode, stream);
+}
+
+extern "C" int bc_encode_kv_into_cache(const void* k, const void* v, void* k_bin, void* k_res, void* v_bin,
+                                       void* v_res, int batch, int seq, int n_heads, int head_dim,
+                                       int start_pos, int max_seq, int scale_mode, int layout,
+                                       void* stream) {
+    BC_REQUIRE(batch >= 0 && n_heads > 0, BC_ERR_INVALID_ARGUMENT, "invalid batch / n_heads");
+    BC_REQUIRE(layout == 0 || layout == 1, BC_ERR_INVALID_ARGUMENT, "layout must be 0 or 1");
+    BC_REQUIRE((k_res == nullptr) == (v_res == nullptr), BC_ERR_INVALID_ARGUMENT,
+               "k_res and v_res must both be given or both be null");
+    const int64_t rows = (int64_t)batch * n_heads;
+    BC_REQUIRE(v != nullptr || rows * seq == 0, BC_ERR_INVALID_ARGUMENT, "null V");
+    return encode_into_cache(k, v, k_bin, k_res, v_bin, v_res, rows, layout == 1 ? n_heads : 1, seq,
+                             head_dim, start_pos, max_seq, scale_mode, stream);
 }

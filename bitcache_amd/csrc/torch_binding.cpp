@@ -287,6 +287,41 @@ void encode_into_cache_bshd(torch::Tensor src, torch::Tensor binary_cache,
                  "encode_into_cache_bshd");
 }
 
+// K and V of a prompt in one launch (bc_encode_kv_into_cache); bshd: sources
+// [batch, seq, n_heads, head_dim], else [batch, n_heads, seq, head_dim].
+void encode_kv_into_cache(torch::Tensor k, torch::Tensor v, torch::Tensor k_bin,
+                          std::optional<torch::Tensor> k_res, torch::Tensor v_bin,
+                          std::optional<torch::Tensor> v_res, int64_t batch, int64_t seq,
+                          int64_t n_heads, int64_t head_dim, int64_t start_pos, int64_t max_seq,
+                          bool fp32_scale, bool bshd) {
+    BC_CHECK_INPUT(k);
+    BC_CHECK_INPUT(v);
+    check_same_device(k, v, "v");
+    check_same_device(k, k_bin, "k_bin");
+    check_same_device(k, v_bin, "v_bin");
+    TORCH_CHECK(k.numel() == batch * seq * n_heads * head_dim && v.numel() == k.numel(),
+                "k and v must hold batch*seq*n_heads*head_dim values");
+    TORCH_CHECK(max_seq > 0 && start_pos >= 0 && start_pos + seq <= max_seq,
+                "start_pos + seq must fit in max_seq");
+    const int64_t cap = batch * n_heads * max_seq;
+    void* kb = blob_exact(k_bin, cap, bc_sizeof_binary_vec(), "k_bin");
+    void* vb = blob_exact(v_bin, cap, bc_sizeof_binary_vec(), "v_bin");
+    TORCH_CHECK(k_res.has_value() == v_res.has_value(), "k_res and v_res: both or neither");
+    void *kr = nullptr, *vr = nullptr;
+    if (k_res.has_value()) {
+        check_same_device(k, *k_res, "k_res");
+        check_same_device(k, *v_res, "v_res");
+        kr = blob_exact(*k_res, cap, bc_sizeof_residual_vec(), "k_res");
+        vr = blob_exact(*v_res, cap, bc_sizeof_residual_vec(), "v_res");
+    }
+    c10::DeviceGuard guard(k.device());
+    check_status(bc_encode_kv_into_cache(k.data_ptr(), v.data_ptr(), kb, kr, vb, vr, (int)batch,
+                                         (int)seq, (int)n_heads, (int)head_dim, (int)start_pos,
+                                         (int)max_seq, fp32_scale ? 1 : 0, bshd ? 1 : 0,
+                                         stream_of(k)),
+                 "encode_kv_into_cache");
+}
+
 // ------------------------------------------------------------------ attention
 void check_q(const torch::Tensor& Q, int64_t batch, int64_t n_heads, int64_t d) {
     BC_CHECK_INPUT(Q);
@@ -641,6 +676,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("encode_into_cache", &encode_into_cache, "Bulk prefill into ring caches");
     m.def("encode_into_cache_bshd", &encode_into_cache_bshd,
           "Bulk prefill into ring caches from a [batch, seq, heads, d] source");
+    m.def("encode_kv_into_cache", &encode_kv_into_cache, "Bulk prefill of K and V in one launch");
     m.def("attention", &attention, "GQA / ring-stride binary or compensated attention");
     m.def("append_attention", &append_attention, "One decode step: ring-cache append + attention");
     m.def("head_mode_attention", &head_mode_attention, "Per-head binary / compensated attention");

@@ -108,6 +108,15 @@ int bc_encode_into_cache_bshd(const void* src, void* binary_cache, void* residua
                               int seq, int n_heads, int head_dim, int start_pos, int max_seq,
                               int scale_mode, void* stream);
 
+/* K and V of a prompt in a single launch, with the bytes of two
+ * bc_encode_into_cache calls (layout 0: k / v [batch, n_heads, seq, head_dim])
+ * or two bc_encode_into_cache_bshd calls (layout 1: [batch, seq, n_heads,
+ * head_dim]).  k_res / v_res: both given or both NULL.  No counterpart in the
+ * reference. */
+int bc_encode_kv_into_cache(const void* k, const void* v, void* k_bin, void* k_res, void* v_bin,
+                            void* v_res, int batch, int seq, int n_heads, int head_dim,
+                            int start_pos, int max_seq, int scale_mode, int layout, void* stream);
+
 /* K and V of one decode step in a single launch (same semantics as two
  * bc_online_encode_token calls).  k_res / v_res may be NULL. */
 int bc_online_encode_kv(const void* k, const void* v, void* k_bin, void* k_res, void* v_bin,

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from oracle import oracle as O
-from tests.gpu_util import (assert_same_bin, assert_same_res, bin_from_blob, res_from_blob, say,
+from tests.gpu_util import (assert_same_bin, assert_same_res, bin_from_blob, res_from_blob, say, slice_enc,
                             to_np)
 
 pytestmark = pytest.mark.gpu
@@ -354,3 +354,40 @@ def test_traffic_probe_stays_in_its_blobs(d, n):
     torch.cuda.synchronize()
     assert torch.all(bfull[n * 36:] == 0xA5) and torch.all(rfull[n * 130:] == 0x5A)
     assert torch.equal(x.view(torch.int16), x0.view(torch.int16))   # bitwise (x holds a NaN)
+
+
+@pytest.mark.parametrize("d", ALL_DIMS)
+def test_kv_prefill_layouts_give_the_same_bytes(d):
+    """K and V of a prompt in one launch, from [B, S, H, d] and [B, H, S, d]
+    sources, write the same cache bytes as the one-tensor calls, at the edges of
+    the encoder's blocked order (positions per wave iteration, blocks of 64
+    positions, ragged ends, fewer positions than an iteration), at an offset
+    in a longer ring, and nothing beside the slots."""
+    from bitcache_amd import _C
+    for B, S, H, start, res in ((1, 3, 5, 0, True), (2, 16, 3, 2, True), (1, 65, 8, 1, True), (2, 511, 2, 0, True),
+                                (1, 512, 3, 7, True), (2, 600, 5, 3, True), (1, 1031, 2, 0, False)):
+        say(f"case kv prefill d={d} B={B} S={S} H={H} start={start} res={res}")
+        g = torch.Generator(device="cuda")
+        g.manual_seed(S + d)
+        max_seq = S + start + 4
+        k, v = (torch.randn((B, H, S, d), generator=g, device="cuda").half() for _ in range(2))
+        kt, vt = (x.transpose(1, 2).contiguous() for x in (k, v))
+        n = B * H * max_seq
+        blobs = lambda: [torch.full((n * per,), 0xA5, dtype=torch.uint8, device="cuda")
+                         for per in (36, 130, 36, 130)]
+        want, got0, got1, one = blobs(), blobs(), blobs(), blobs()
+        opt = lambda b: (b[0], b[1] if res else None, b[2], b[3] if res else None)
+        for src, bin_, r in ((k, want[0], want[1]), (v, want[2], want[3])):
+            _C.encode_into_cache(src, bin_, r if res else None, B * H, S, d, start, max_seq, True)
+        for src, bin_, r in ((kt, one[0], one[1]), (vt, one[2], one[3])):
+            _C.encode_into_cache_bshd(src, bin_, r if res else None, B, S, H, d, start, max_seq, True)
+        _C.encode_kv_into_cache(k, v, *opt(got0), B, S, H, d, start, max_seq, True, False)
+        _C.encode_kv_into_cache(kt, vt, *opt(got1), B, S, H, d, start, max_seq, True, True)
+        for name, got in (("bshd", one), ("kv bhsd", got0), ("kv bshd", got1)):
+            for x, y in zip(got, want):
+                assert torch.equal(x, y), f"{name} d={d} S={S}"
+        # and the oracle's bytes, for the first row of K
+        O_b, O_r = O.online_encode(to_np(k[0, 0]))
+        assert_same_bin(slice_enc(bin_from_blob(want[0], n, d), start, start + S), O_b, f"d={d} S={S}")
+        if res:
+            assert_same_res(slice_enc(res_from_blob(want[1], n, d), start, start + S), O_r, f"d={d} S={S}")
