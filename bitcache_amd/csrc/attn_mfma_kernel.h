@@ -18,8 +18,8 @@
 // int8 path (groups up to 4; I8 and R8 below): sign bits in place as int8
 // elements, codes as 16 n, four keys per operation, the weights of each head
 // as balanced 8-bit digit columns, v_mfma_i32_16x16x64_i8 with exact int32
-// sums, flushed into a float bank on rescales.  fp16 path (groups of 8, and
-// the adaptive mode's residuals): nibbles (u = n + 8, the 8 b_s taken off at
+// sums, flushed into a float bank on rescales.  fp16 path (groups of 8):
+// nibbles (u = n + 8, the 8 b_s taken off at
 // the end) and sign bits become exact fp16 subnormals (value * 2^(j-24) for
 // bit position j < 10) with one mask per pair of keys, left in place (the
 // power of two is folded into the weights of odd keys and into the
@@ -151,8 +151,7 @@ struct WaveLds {
     // weight columns of 72 slots (64 used): the 16 lanes of a row group read
     // 16-byte runs of 16 columns without LDS bank conflicts
     static constexpr int kColSlots = 72;
-    // (one part where the int8 path holds the other)
-    static constexpr int kWeightBytes = (G <= 4 ? 1 : 2) * 2 * G * kColSlots * 2;
+    static constexpr int kWeightBytes = 2 * 2 * G * kColSlots * 2;
     static constexpr int kRdInts = KMF ? 64 * G : 4;
     // epilogue: heads per pass through staging buffer 0 ([parts][heads][D] floats)
     static constexpr int kEpiHeads = kStage / ((RES ? 2 : 1) * D * 4) < G ? kStage / ((RES ? 2 : 1) * D * 4) : G;
@@ -525,15 +524,14 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
     // word.  The sums are exact in int32 accumulators.  A rescale (running max
     // or weight plan) flushes them, scaled, into a per-wave float bank in LDS
     // and restarts them at zero (flush8).
-    // R8: the residual part too (every mode but adaptive, whose residual
-    // positions are compacted): a code n enters as 16 n, eight codes in three
+    // R8: the residual part too.  A code n enters as 16 n, eight codes in three
     // operations, its weight as digits of the same kind, and no offset is
     // needed for the codes' sign (fp16 codes are n + 8).  The sums are exact,
     // where fp32 accumulation in the matrix cores drops low bits of every
     // partial sum (the fp16 path at unit variance: 2.6e-4 to 2.9e-4 of the
     // output against 64 bits; the fp16 output's own rounding is 2.1e-4).
     constexpr bool I8 = G <= 4;
-    constexpr bool R8 = I8 && ALLRES;
+    constexpr bool R8 = I8 && RES;
     // int8 weights in LDS: a row per slot, 4 digit bytes per head (and part),
     // read back as columns by ds_read_b64_tr_b8 (16-byte rows; a shorter row
     // is read twice, its columns repeating).  Up to two heads, one row holds
@@ -548,7 +546,7 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
     __shared__ QDigits<D, G, KMF> qd;
     __shared__ __attribute__((aligned(16))) uint8_t lds_st0[NW][WL::kStage];
     __shared__ __attribute__((aligned(16))) uint8_t lds_st1[NW][PIPE ? WL::kStage : 16];
-    __shared__ __attribute__((aligned(16))) uint16_t lds_wts[NW][(I8 && MODE != MODE_ADAPTIVE) ? 8 : WL::kWeightBytes / 2];
+    __shared__ __attribute__((aligned(16))) uint16_t lds_wts[NW][I8 ? 8 : WL::kWeightBytes / 2];
     __shared__ __attribute__((aligned(16))) uint8_t lds_w8[NW][I8 ? 64 * kWRow : 16];
     // (int8 path) per wave and head, the float sums of the keys before the
     // last rescale, [head][D]
@@ -855,7 +853,7 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
     int* rdl = lds_rd[wave];          // [64 keys][G] residual dots
     int* rdlo = lds_rdlo[wave];       // their plane-0 parts (precise tiles)
 
-    constexpr int kRes0 = I8 ? 0 : 2 * G;   // first fp16 residual weight column
+    constexpr int kRes0 = 2 * G;   // first fp16 residual weight column
     // softmax reference per head, lowered lazily: weights p = 2^(s - m) stay
     // <= 2^kTau, and the accumulators are rescaled only when a score passes
     // m + kTau (the result does not depend on m)
@@ -1330,7 +1328,6 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
 
         // online softmax; (hi, lo) fp16 weights to LDS in MFMA slot order
         float lane_alpha = 1.0f;
-        float lane_ralpha = 1.0f;   // (int8 path) the residual part's head
         bool any_rescale = false;
         // the value operands of odd rows come out 16x larger (see the MFMA
         // loops below): their weights carry 1/16 so that every product is exact
@@ -1341,8 +1338,7 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
         // per-key factors shared by the heads: sign weight a2 = p * fa, residual
         // weight b = p * fb, and the offset sum_s (a_s + 8 b_s) grows by p * fo
         const float fa = ldexpf(2.0f * svv * kfac, wexp);
-        // (adaptive: the fp16 residual weights stay below 2^14 at 2^(wexp - 16))
-        const float fb = RES ? ldexpf(rsv * (1.0f / 7.0f) * kfac_res, wexp - (R8 ? 0 : kWTop - 14)) : 0.0f;
+        const float fb = RES ? ldexpf(rsv * (1.0f / 7.0f) * kfac_res, wexp) : 0.0f;
         const float fo_bin = ldexpf(svv, wexp);
         // (int8 codes need no offset; a V scale that is not finite has no
         // integer weight, and makes the offset, so the output, NaN)
@@ -1351,11 +1347,14 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
         // (adaptive: compacted; unselected keys write zeros to the positions
         // past nsel, so every slot a residual MFMA reads is written)
         uint16_t* wres = wsl;
+        uint8_t* w8res = w8st;
         uint32_t dsig[G], dres[G];   // (int8 path) packed digits
         // the weight p * f <= 2^30, rounded (weights are not negative), as
         // balanced digits
         auto pack8 = [](float p, float f) { return ((uint32_t)(int)fmaf(p, f, 0.5f) + 0x80808080u) ^ 0x80808080u; };
-        if constexpr (MODE == MODE_ADAPTIVE)
+        if constexpr (MODE == MODE_ADAPTIVE && I8)
+            w8res = &lds_w8[0][0] + opaque_int((wave * 64 + slot8_of(res_row(rpos))) * kWRow);
+        else if constexpr (MODE == MODE_ADAPTIVE)
             wres = &lds_wts[0][0] + opaque_int(wave * (WL::kWeightBytes / 2) + slot_of(res_row(rpos)));
 #pragma unroll
         for (int g = 0; g < G; g++) {
@@ -1366,7 +1365,6 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
                 lsum[g] *= alpha;
                 off[g] *= alpha;
                 if (my_head == g) lane_alpha = alpha;
-                if (I8 && my_rhead == g) lane_ralpha = alpha;
                 any_rescale = true;
                 m[g] = mn;
                 mlim[g] = mn + kTau;
@@ -1402,13 +1400,21 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
         }
         if constexpr (I8 && G == 4) {
             *(v4u_t*)w8st = v4u_t{dsig[0], dsig[1], dsig[2], dsig[3]};
-            if constexpr (R8) *(v4u_t*)(w8st + 16) = v4u_t{dres[0], dres[1], dres[2], dres[3]};
+            if constexpr (R8) *(v4u_t*)(w8res + 16) = v4u_t{dres[0], dres[1], dres[2], dres[3]};
         } else if constexpr (I8 && G == 2) {
-            if constexpr (R8) *(v4u_t*)w8st = v4u_t{dsig[0], dsig[1], dres[0], dres[1]};
-            else *(v2u_t*)w8st = v2u_t{dsig[0], dsig[1]};
+            if constexpr (R8 && ALLRES) {
+                *(v4u_t*)w8st = v4u_t{dsig[0], dsig[1], dres[0], dres[1]};
+            } else {
+                *(v2u_t*)w8st = v2u_t{dsig[0], dsig[1]};
+                if constexpr (R8) *(v2u_t*)(w8res + 8) = v2u_t{dres[0], dres[1]};
+            }
         } else if constexpr (I8) {
-            if constexpr (R8) *(v2u_t*)w8st = v2u_t{dsig[0], dres[0]};
-            else *(uint32_t*)w8st = dsig[0];
+            if constexpr (R8 && ALLRES) {
+                *(v2u_t*)w8st = v2u_t{dsig[0], dres[0]};
+            } else {
+                *(uint32_t*)w8st = dsig[0];
+                if constexpr (R8) *(uint32_t*)(w8res + 4) = dres[0];
+            }
         }
         if constexpr (I8) {
             // the integer sums so far move to the float bank, scaled by this
@@ -1416,11 +1422,6 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
             // passed m + kTau, or the residual sums are full)
             if (live8 > 0 && (any_rescale || wfac != 1.0f || (R8 && live8 >= kMaxTiles8)))
                 flush8(lane_alpha * wfac);
-            if (RES && !R8 && any_rescale) {
-                if (my_rhead >= G) lane_ralpha = 1.0f;
-#pragma unroll
-                for (int d = 0; d < NB; d++) cn[d] *= lane_ralpha;
-            }
         } else if (any_rescale) {
             if (my_head >= G) lane_alpha = 1.0f;
 #pragma unroll
@@ -1470,10 +1471,6 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
             b8 = columns(w8rd);
             b8r = b8;
             if constexpr (R8 && G == 4) b8r = columns(w8rd + 16);
-            if constexpr (RES && !R8) {
-#pragma unroll
-                for (int mh = 0; mh < 2; mh++) bres[mh] = *(const h8_t*)&wrd[kRes0 * WL::kColSlots + 8 * mh];
-            }
         } else {
 #pragma unroll
             for (int mh = 0; mh < 2; mh++) {
@@ -1558,7 +1555,21 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
             const h8_t av = __builtin_bit_cast(h8_t, pw);
             cn[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bres[mh], cn[db], 0, 0, 0);
         };
-        if constexpr (MODE == MODE_ADAPTIVE) {
+        if constexpr (MODE == MODE_ADAPTIVE && R8) {
+            // positions 0..31 are the first words, the second ones only past 32
+            if (nmh == 1) {
+#pragma unroll
+                for (int db = 0; db < NB; db++) {
+                    const uint32_t x = (uint32_t)wrs[db].x;
+                    const v4i_t av = v4i_t{(int)((x << 4) & 0xF0F0F0F0u), (int)(x & 0xF0F0F0F0u), 0, 0};
+                    cr[db] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, b8r, cr[db], 0, 0, 0);
+                }
+            } else if (nmh == 2) {
+#pragma unroll
+                for (int db = 0; db < NB; db++)
+                    cr[db] = __builtin_amdgcn_mfma_i32_16x16x64_i8(codes_i8((uint32_t)wrs[db].x, (uint32_t)wrs[db].y), b8r, cr[db], 0, 0, 0);
+            }
+        } else if constexpr (MODE == MODE_ADAPTIVE) {
             // half 0 when any key is selected, half 1 only past 32 of them
 #pragma unroll
             for (int mh = 0; mh < 2; mh++) {
@@ -1694,7 +1705,6 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
     for (int g0 = 0; g0 < G; g0 += HP) {
         const int hs = my_head - g0;   // this lane's head slot in the batch
         const bool wr = writer && hs >= 0 && hs < HP;
-        // the residual part's writer (adaptive: in the fp16 column layout)
         const int rhs = my_rhead - g0;
         const bool rwr = (R8 ? rowner8 : my_col < 2 * G && (my_col & 1) == 0) && rhs >= 0 && rhs < HP;
         if (g0 > 0) __syncthreads();   // the previous batch has been read
@@ -1756,14 +1766,12 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
             }
         }
         if constexpr (RES) {
-            // (adaptive: the residual part's units of 2^-24, its weights 2^-16
-            // of the sign weights' scale, become the sign part's units)
             if (rwr) {
 #pragma unroll
                 for (int d = 0; d < NB; d++)
 #pragma unroll
                     for (int i = 0; i < 4; i++)
-                        accw[(1 * HP + rhs) * D + 16 * d + 4 * g4 + i] = I8 && !R8 ? nv[d][i] * (two24 * 65536.0f) : nv[d][i];
+                        accw[(1 * HP + rhs) * D + 16 * d + 4 * g4 + i] = nv[d][i];
             }
         }
         __syncthreads();
