@@ -890,7 +890,22 @@ struct SplitPlan {
 // per-CU speed differences of a long bandwidth-bound launch (measured faster
 // on the 64K-context MHA compensated step); a launch too small for two such
 // rounds fills one round of 3 workgroups per CU.
+//
+// Short launches (at two workgroups per CU no wave takes more than kShortTiles
+// tiles) run one round of at most two workgroups per CU instead: there a
+// workgroup's fixed work counts against its few tiles, and three of them
+// share the CU's issue slots, so the plan that costs least is the one whose
+// waves take whole numbers of tiles (4x(32/8) heads of 16384 keys, append +
+// attend: 24 splits 26.7 us, 16 splits 24.8; binary 4x(32/8) heads of 16000
+// keys: 32 splits 17.5 us, 16 splits 15.4; 18601 keys, five tiles per wave at
+// two per CU: 24 splits 25.5, 16 splits 26.2, so it keeps its round of three).
+// per_cu = kPlanMha: as 0, but the launches too small for two rounds of eight
+// fill one of two workgroups per CU (4x16 heads of 9300 keys 24.5 -> 23.3 us,
+// 2x32 heads of 9973 keys, d = 96, 22.5 -> 21.2).
 // `cu` is the device's CU count (0: the current device's).
+constexpr int kMaxPerCu = 4;
+constexpr int kPlanMha = kMaxPerCu + 1;
+constexpr int kShortTiles = 4;   // per wave
 SplitPlan plan_splits(int batch, int hq, int hkv, int S, int per_cu, int cu = 0) {
     SplitPlan p;
     p.G = pick_g(hq / hkv);
@@ -900,8 +915,14 @@ SplitPlan plan_splits(int batch, int hq, int hkv, int S, int per_cu, int cu = 0)
     int max_split = tiles / 8;                   // at least 8 tiles (2 per wave) per split
     if (max_split > kMaxSplits) max_split = kMaxSplits;   // the combine kernel's weight table
     if (max_split < 1) max_split = 1;
+    // ... and one per wave while every workgroup has a CU to itself (32/8
+    // heads of 4096 keys: 8 splits 12.9 us, 16 splits 11.8)
+    if (groups > 0 && groups * max_split < cu) {
+        const int64_t alone = cu / groups < tiles / 4 ? cu / groups : tiles / 4;
+        if (alone > max_split) max_split = alone < kMaxSplits ? (int)alone : kMaxSplits;
+    }
     int want = 1;
-    if (groups > 0 && tiles > 0 && per_cu > 0) {
+    if (groups > 0 && tiles > 0 && per_cu > 0 && per_cu <= kMaxPerCu) {
         const int64_t slots = (int64_t)per_cu * cu;
         // beyond 4 rounds' worth of splits nothing improves
         const int64_t lim = 4 * slots / groups + 1;
@@ -918,11 +939,29 @@ SplitPlan plan_splits(int batch, int hq, int hkv, int S, int per_cu, int cu = 0)
                 want = sp;
             }
         }
+        // a short launch: the fewest tiles per wave times the workgroups that
+        // share a CU, among the plans of one or two per CU
+        const int64_t two = 2LL * cu / groups < max_split ? 2LL * cu / groups : max_split;
+        if (per_cu >= 2 && two >= 1 && (tiles + 4 * two - 1) / (4 * two) <= kShortTiles &&
+            groups * want > 2LL * cu) {
+            int64_t least = 0;
+            for (int sp = 1; sp <= two; sp++) {
+                const int per = (tiles + sp - 1) / sp;
+                if ((tiles + per - 1) / per != sp) continue;
+                const int64_t w = (groups * sp + cu - 1) / cu;
+                // (one workgroup alone on a CU waits for its own latencies: 7/4)
+                const int64_t t = (int64_t)((per + 3) / 4) * (w == 1 ? 7 : 4 * w) + 5 * w;
+                if (least == 0 || t < least) {
+                    least = t;
+                    want = sp;
+                }
+            }
+        }
     } else if (groups > 0) {
         want = (int)((8 * cu + groups - 1) / groups);
         if (want > max_split) want = max_split;
         if (groups * want < 6LL * cu) {
-            const int64_t one_round = (3LL * cu) / groups;
+            const int64_t one_round = ((per_cu == kPlanMha ? 2LL : 3LL) * cu) / groups;
             want = one_round < max_split ? (int)one_round : max_split;
         }
     }
@@ -946,14 +985,14 @@ SplitPlan plan_splits(int batch, int hq, int hkv, int S, int per_cu, int cu = 0)
 // at most two (its tiles are short, so a workgroup's fixed prologue and
 // epilogue weigh more than the latency hiding of a third: c2 54.5 -> 52.9 us).
 //
-// kMaxPerCu bounds every policy: ws_bytes sizes the workspace over the plans
-// of per_cu = 0 .. kMaxPerCu, so a policy above it would launch more splits
+// kPlanMha bounds every policy: ws_bytes sizes the workspace over the plans
+// of per_cu = 0 .. kPlanMha, so a policy above it would launch more splits
 // than the workspace holds.
-constexpr int kMaxPerCu = 4;
 int plan_per_cu(int mode, int D, int G) {
-    if ((mode == MODE_COMP || mode == MODE_MIXED) && G == 1) return 0;
-    // (MHA binary 2, GQA binary 4, the other modes 3: measured)
-    int cap = mode == MODE_BINARY ? (G == 1 ? 2 : 4) : 3;
+    if ((mode == MODE_COMP || mode == MODE_MIXED) && G == 1) return kPlanMha;
+    // (MHA binary 2, GQA binary 4, the other modes 3, and 4 up to d = 64,
+    // where four workgroups fit: 8x(32/8) heads of 20011 keys 26.8 -> 25.7 us)
+    int cap = mode == MODE_BINARY ? (G == 1 ? 2 : 4) : (D <= 64 ? 4 : 3);
     if (cap > kMaxPerCu) cap = kMaxPerCu;
     const int n = bc::mfma_wgs_per_cu(mode, D, G);
     return n <= 0 ? cap : (n < cap ? n : cap);
@@ -1012,10 +1051,10 @@ size_t list_offset(size_t partial_bytes) { return (partial_bytes + 255) & ~(size
 size_t list_bytes(int64_t groups) { return kListHeader + 2 * (size_t)groups * sizeof(int32_t); }
 
 // workspace of the split partials: the largest plan of any policy
-// plan_per_cu can return (per_cu = 0 .. kMaxPerCu), and the group lists
+// plan_per_cu can return (per_cu = 0 .. kPlanMha), and the group lists
 size_t ws_bytes(int batch, int hq, int hkv, int S, int D, int cu = 0) {
     size_t n = plan_bytes(batch, hq, plan_splits(batch, hq, hkv, S, 0, cu), D);
-    for (int per_cu = 1; per_cu <= kMaxPerCu; per_cu++) {
+    for (int per_cu = 1; per_cu <= kPlanMha; per_cu++) {
         const size_t b = plan_bytes(batch, hq, plan_splits(batch, hq, hkv, S, per_cu, cu), D);
         n = b > n ? b : n;
     }
