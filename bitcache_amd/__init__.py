@@ -169,9 +169,10 @@ class BitCache:
         assert self._filled > 0, "cache is empty, call append() first"
         assert (threshold is None) != (modes is None), "give exactly one of threshold and modes"
         if modes is None:
-            ent = _C.head_entropy(Q, self._k_bin, self.batch, self.n_heads, self.n_kv_heads,
-                                  self._filled, self.max_seq, self.head_dim)
-            modes = _C.adaptive_select(ent, threshold).view(self.batch, self.n_heads)
+            out, modes = _C.entropy_dispatch_attention(
+                Q, self._k_bin, self._k_res, self._v_bin, self._v_res, self.batch, self.n_heads,
+                self.n_kv_heads, self._filled, self.max_seq, self.head_dim, threshold)
+            return (out, modes) if return_modes else out
         out = _C.head_mode_attention(Q, self._k_bin, self._k_res, self._v_bin, self._v_res,
                                      modes.contiguous(), self.batch, self.n_heads,
                                      self.n_kv_heads, self._filled, self.max_seq, self.head_dim)

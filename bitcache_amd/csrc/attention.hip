@@ -703,28 +703,30 @@ __global__ __launch_bounds__(T) void entropy_kernel(const uint16_t* q, BinPlanes
                                                     float* ws, int Hq, int Hkv, int S,
                                                     int kv_stride, int chunk) {
     constexpr int NW = T / 64;
-    __shared__ float part[128];
-    __shared__ uint32_t qs[D / 32];
     __shared__ float sm[NW], sz[NW], sw[NW];
     const int bh = blockIdx.x, c = blockIdx.y;
     const uint16_t* qb = q + (int64_t)bh * D;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid < 128) {
-        float local = 0.0f;
-        for (int i = tid; i < D; i += 128) local += fabsf(h2f(qb[i]));
-        part[tid] = local;
+    // every wave forms the query's sign words (ballots) and scale itself, with
+    // no barrier: lane l is threads l and l + 64 of the reference's 128 (s = 64
+    // in the lane), and the xor butterfly's lane-0 sum has the tree's
+    // association (fp32 addition commutes)
+    uint32_t qs[D / 32];
+    float pa = 0.0f, pb = 0.0f;
+#pragma unroll
+    for (int k = 0; k < (D + 63) / 64; k++) {
+        const int e = lane + 64 * k;
+        const float x = e < D ? h2f(qb[e]) : 0.0f;
+        const uint64_t bits = __ballot(x >= 0.0f);
+        qs[2 * k] = (uint32_t)bits;
+        if (2 * k + 1 < D / 32) qs[2 * k + 1] = (uint32_t)(bits >> 32);
+        if (k % 2 == 0) pa += fabsf(x);
+        else pb += fabsf(x);
     }
-    if (tid < D / 32) {
-        uint32_t bits = 0;
-        for (int i = 0; i < 32; i++) bits |= (h2f(qb[32 * tid + i]) >= 0.0f ? 1u : 0u) << i;
-        qs[tid] = bits;
-    }
-    __syncthreads();
-    for (int st = 64; st > 0; st >>= 1) {
-        if (tid < st) part[tid] += part[tid + st];
-        __syncthreads();
-    }
-    const float sq = part[0] / (float)D;
+    float tree = pa + pb;
+#pragma unroll
+    for (int st = 32; st > 0; st >>= 1) tree = tree + __shfl_xor(tree, st, 64);
+    const float sq = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, tree))) / (float)D;
     // query head h of batch b reads kv head h / (Hq / Hkv) of that batch
     const int b = bh / Hq, kvh = (bh % Hq) / (Hq / Hkv);
     const int64_t base = ((int64_t)b * Hkv + kvh) * kv_stride;
@@ -797,10 +799,8 @@ __global__ __launch_bounds__(T) void entropy_kernel(const uint16_t* q, BinPlanes
     }
 }
 
-// H per (b, h) from its nchunk (M, Z, W) partials (one thread per head)
-__global__ void entropy_merge_kernel(const float* ws, float* out, int n, int nchunk) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+// H of head i from its nchunk (M, Z, W) partials
+__device__ __forceinline__ float merged_entropy(const float* ws, int i, int nchunk) {
     const float* p = ws + (int64_t)i * nchunk * 3;
     float gm = -1e30f;
     for (int c = 0; c < nchunk; c++) gm = fmaxf(gm, p[3 * c]);
@@ -810,21 +810,45 @@ __global__ void entropy_merge_kernel(const float* ws, float* out, int n, int nch
         z += p[3 * c + 1] * f;
         w += p[3 * c + 2] * f;
     }
-    out[i] = (logf(z) + gm) - w / fmaxf(z, 1e-12f);
+    return (logf(z) + gm) - w / fmaxf(z, 1e-12f);
+}
+
+// one thread per head
+__global__ void entropy_merge_kernel(const float* ws, float* out, int n, int nchunk) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = merged_entropy(ws, i, nchunk);
 }
 
 // Query-head groups of per-head modes, compacted in order: group y (heads
 // b*Hq + hq0 .. + G - 1 of grid row y, as the attention kernels map it) goes
 // to the binary list when all its heads have mode 0, else to the mixed list.
 // One block; lists[0], lists[1] = the counts, the lists from word 64 on.
+// DISPATCH: the modes come from the heads' entropies first (mode 0 where H >=
+// thr, written to head_mode): entropy merge, selection and lists in one launch
+// instead of three of a few microseconds each (per-head modes of 4x32 heads of
+// 16384 keys: 68.5 -> 63.2 us with the entropy pass's shorter prologue).
+struct DispatchArgs {
+    const float* entropy;   // [n] entropies, or (nchunk > 1) the chunk partials
+    int nchunk, n;          // chunks per head, heads
+    float thr;
+};
 constexpr int kListThreads = 1024;
 constexpr size_t kListHeader = 256;   // bytes before the lists (the two counts)
-__global__ __launch_bounds__(kListThreads) void mode_groups_kernel(const uint8_t* head_mode,
+template <bool DISPATCH>
+__global__ __launch_bounds__(kListThreads) void mode_groups_kernel(uint8_t* head_mode,
                                                                    int32_t* lists, int groups,
-                                                                   int nqg, int Hq, int Hkv,
-                                                                   int G) {
+                                                                   int G, DispatchArgs d) {
     __shared__ int wb[kListThreads / 64], wm_[kListThreads / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if constexpr (DISPATCH) {
+        for (int i = tid; i < d.n; i += kListThreads) {
+            const float h = d.nchunk > 1 ? merged_entropy(d.entropy, i, d.nchunk) : d.entropy[i];
+            head_mode[i] = h >= d.thr ? 0 : 1;   // src/adaptive_precision.cu:133-144
+        }
+        // (the block reads its own stores below)
+        __threadfence_block();
+        __syncthreads();
+    }
     int32_t* bin_list = lists + kListHeader / sizeof(int32_t);
     int32_t* mix_list = bin_list + groups;
     int nb = 0, nm = 0;   // entries written so far (uniform)
@@ -832,10 +856,7 @@ __global__ __launch_bounds__(kListThreads) void mode_groups_kernel(const uint8_t
         const int y = y0 + tid;
         bool live = y < groups, res = false;
         if (live) {
-            const int qg = y % nqg, bkv = y / nqg;
-            const int b = bkv / Hkv, kvh = bkv % Hkv;
-            const int bhq0 = b * Hq + kvh * (Hq / Hkv) + qg * G;
-            for (int g = 0; g < G; g++) res |= head_mode[bhq0 + g] != 0;
+            for (int g = 0; g < G; g++) res |= head_mode[y * G + g] != 0;   // (group y: heads G y ..)
         }
         const uint64_t mb = __ballot(live && !res), mm = __ballot(live && res);
         const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -1127,7 +1148,7 @@ int run_partial(int mode, const void* q, const void* k_bin, const void* k_res, c
                 hipStream_t st, const uint32_t* thresh, const int32_t* cutoff,
                 uint8_t* selected, const void* pcs, int per_cu, const AppendArgs* app = nullptr,
                 const uint8_t* head_mode = nullptr, void* direct_out = nullptr,
-                bool* wrote_out = nullptr) {
+                bool* wrote_out = nullptr, const DispatchArgs* dispatch = nullptr) {
     if (wrote_out) *wrote_out = false;
     int v = validate_heads(batch, n_heads, n_kv_heads, seq_len, kv_stride, head_dim);
     if (v != BC_OK) return v;
@@ -1188,9 +1209,13 @@ int run_partial(int mode, const void* q, const void* k_bin, const void* k_res, c
     int32_t* lists = nullptr;
     if (mode == MODE_MIXED) {
         lists = (int32_t*)((uint8_t*)workspace + list_offset(plan_ws));
-        hipLaunchKernelGGL(mode_groups_kernel, dim3(1), dim3(kListThreads), 0, st, head_mode,
-                           lists, (int)groups, (n_heads / n_kv_heads) / p.G, n_heads, n_kv_heads,
-                           p.G);
+        // (head_mode is written only with a dispatch, whose modes it receives)
+        if (dispatch != nullptr)
+            hipLaunchKernelGGL((mode_groups_kernel<true>), dim3(1), dim3(kListThreads), 0, st,
+                               (uint8_t*)head_mode, lists, (int)groups, p.G, *dispatch);
+        else
+            hipLaunchKernelGGL((mode_groups_kernel<false>), dim3(1), dim3(kListThreads), 0, st,
+                               (uint8_t*)head_mode, lists, (int)groups, p.G, DispatchArgs{});
         const int rc = bc::check_launch("per-head mode groups");
         if (rc != BC_OK) return rc;
         a.group_list = lists + kListHeader / sizeof(int32_t);
@@ -1246,12 +1271,32 @@ int run_combine(int per_cu, const void* workspace, void* out, int batch, int n_h
     return bc::check_launch("attention combine");
 }
 
+static int run_attention_dispatch(int mode, const void* q, const void* k_bin, const void* k_res,
+                                  const void* v_bin, const void* v_res, void* out, int batch, int n_heads,
+                                  int n_kv_heads, int seq_len, int kv_stride, int head_dim,
+                                  void* workspace, size_t workspace_bytes, hipStream_t st,
+                                  const uint32_t* thresh, const int32_t* cutoff, uint8_t* selected,
+                                  const void* pcs, const AppendArgs* app, const uint8_t* head_mode,
+                                  const DispatchArgs* dispatch);
+
 int run_attention(int mode, const void* q, const void* k_bin, const void* k_res, const void* v_bin,
                   const void* v_res, void* out, int batch, int n_heads, int n_kv_heads,
                   int seq_len, int kv_stride, int head_dim, void* workspace,
                   size_t workspace_bytes, hipStream_t st, const uint32_t* thresh,
                   const int32_t* cutoff, uint8_t* selected, const void* pcs, const AppendArgs* app,
                   const uint8_t* head_mode) {
+    return run_attention_dispatch(mode, q, k_bin, k_res, v_bin, v_res, out, batch, n_heads, n_kv_heads,
+                                  seq_len, kv_stride, head_dim, workspace, workspace_bytes, st, thresh,
+                                  cutoff, selected, pcs, app, head_mode, nullptr);
+}
+
+static int run_attention_dispatch(int mode, const void* q, const void* k_bin, const void* k_res,
+                                  const void* v_bin, const void* v_res, void* out, int batch, int n_heads,
+                                  int n_kv_heads, int seq_len, int kv_stride, int head_dim,
+                                  void* workspace, size_t workspace_bytes, hipStream_t st,
+                                  const uint32_t* thresh, const int32_t* cutoff, uint8_t* selected,
+                                  const void* pcs, const AppendArgs* app, const uint8_t* head_mode,
+                                  const DispatchArgs* dispatch) {
     const int per_cu = head_dim > 0 && n_kv_heads > 0
                            ? plan_per_cu(mode, head_dim, pick_g(n_heads / n_kv_heads)) : kPlanFixed;
     BC_REQUIRE(out != nullptr || (int64_t)batch * n_heads == 0, BC_ERR_INVALID_ARGUMENT,
@@ -1259,7 +1304,7 @@ int run_attention(int mode, const void* q, const void* k_bin, const void* k_res,
     bool wrote = false;
     int rc = run_partial(mode, q, k_bin, k_res, v_bin, v_res, batch, n_heads, n_kv_heads, seq_len,
                          kv_stride, head_dim, workspace, workspace_bytes, st, thresh, cutoff,
-                         selected, pcs, per_cu, app, head_mode, out, &wrote);
+                         selected, pcs, per_cu, app, head_mode, out, &wrote, dispatch);
     if (rc != BC_OK || wrote) return rc;
     return run_combine(per_cu, workspace, out, batch, n_heads, n_kv_heads, seq_len, head_dim, st);
 }
@@ -1512,7 +1557,7 @@ static size_t entropy_ws_bytes(int batch, int hq, int S) {
 
 template <int D>
 static void launch_entropy(const void* q, BinPlanes kb, float* out, float* ws, int batch, int hq,
-                           int hkv, int S, int stride, hipStream_t st) {
+                           int hkv, int S, int stride, hipStream_t st, bool merge) {
     const int n = ws != nullptr ? entropy_chunks(batch, hq, S) : 1;
     if (n <= 1) {
         hipLaunchKernelGGL((entropy_kernel<D, kEntropyThreads>), dim3(batch * hq, 1),
@@ -1524,6 +1569,7 @@ static void launch_entropy(const void* q, BinPlanes kb, float* out, float* ws, i
     hipLaunchKernelGGL((entropy_kernel<D, kEntPartThreads>), dim3(batch * hq, n),
                        dim3(kEntPartThreads), 0, st, (const uint16_t*)q, kb, out, ws, hq, hkv, S,
                        stride, chunk);
+    if (!merge) return;
     const int heads = batch * hq;
     hipLaunchKernelGGL(entropy_merge_kernel, dim3((heads + 255) / 256), dim3(256), 0, st,
                        (const float*)ws, out, heads, n);
@@ -1552,8 +1598,54 @@ extern "C" int bc_compute_head_entropy_ws(const void* q, const void* k_bin, floa
     BinPlanes kb = bin_planes(k_bin, cap, head_dim);
     float* ws = need > 0 ? (float*)workspace : nullptr;
     BC_DISPATCH_D(head_dim, launch_entropy, q, kb, entropy, ws, batch, n_heads, n_kv_heads,
-                  seq_len, kv_stride, (hipStream_t)stream);
+                  seq_len, kv_stride, (hipStream_t)stream, true);
     return bc::check_launch("entropy");
+}
+
+// Entropy pass into `ws` (chunk partials, or the entropies themselves when a
+// head is one chunk), then the per-head launches with the modes selected in
+// the list kernel.
+extern "C" int bc_entropy_dispatch_workspace_size(int batch, int n_heads, int n_kv_heads, int seq_len,
+                                                  int head_dim, size_t* bytes) {
+    int v = validate_heads(batch, n_heads, n_kv_heads, seq_len, seq_len, head_dim);
+    if (v != BC_OK) return v;
+    BC_REQUIRE(bytes != nullptr, BC_ERR_INVALID_ARGUMENT, "null bytes");
+    const size_t attn = ws_bytes(batch, n_heads, n_kv_heads, seq_len, head_dim);
+    const size_t ent = entropy_ws_bytes(batch, n_heads, seq_len);
+    *bytes = list_offset(attn) + (ent > 0 ? ent : (size_t)batch * n_heads * sizeof(float));
+    return BC_OK;
+}
+
+extern "C" int bc_entropy_dispatch_attention(const void* q, const void* k_bin, const void* k_res,
+                                             const void* v_bin, const void* v_res, uint8_t* modes,
+                                             void* out, int batch, int n_heads, int n_kv_heads,
+                                             int seq_len, int kv_stride, int head_dim, float threshold,
+                                             void* workspace, size_t workspace_bytes, void* stream) {
+    int v = validate_heads(batch, n_heads, n_kv_heads, seq_len, kv_stride, head_dim);
+    if (v != BC_OK) return v;
+    if ((int64_t)batch * n_heads == 0) return BC_OK;
+    BC_REQUIRE(q && k_bin && k_res && v_bin && v_res && modes && out, BC_ERR_INVALID_ARGUMENT,
+               "null pointer");
+    size_t need = 0;
+    v = bc_entropy_dispatch_workspace_size(batch, n_heads, n_kv_heads, seq_len, head_dim, &need);
+    if (v != BC_OK) return v;
+    BC_REQUIRE(workspace != nullptr && workspace_bytes >= need, BC_ERR_WORKSPACE,
+               "workspace of %zu bytes required, got %zu", need, workspace_bytes);
+    const size_t attn = list_offset(ws_bytes(batch, n_heads, n_kv_heads, seq_len, head_dim));
+    float* ent = (float*)((uint8_t*)workspace + attn);
+    const int64_t cap = (int64_t)batch * n_kv_heads * kv_stride;
+    BinPlanes kb = bin_planes(k_bin, cap, head_dim);
+    const int nchunk = entropy_chunks(batch, n_heads, seq_len);
+    const bool partials = nchunk > 1;
+    BC_DISPATCH_D(head_dim, launch_entropy, q, kb, ent, partials ? ent : nullptr, batch, n_heads,
+                  n_kv_heads, seq_len, kv_stride, (hipStream_t)stream, false);
+    v = bc::check_launch("entropy");
+    if (v != BC_OK) return v;
+    const DispatchArgs d{ent, nchunk, batch * n_heads, threshold};
+    return bc::run_attention_dispatch(MODE_MIXED, q, k_bin, k_res, v_bin, v_res, out, batch, n_heads,
+                                      n_kv_heads, seq_len, kv_stride, head_dim, workspace, attn,
+                                      (hipStream_t)stream, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                      modes, &d);
 }
 
 extern "C" int bc_compute_head_entropy_gqa(const void* q, const void* k_bin, float* entropy,

@@ -414,6 +414,32 @@ torch::Tensor head_mode_attention(torch::Tensor Q, torch::Tensor K_bin, torch::T
     return out.view(Q.sizes());
 }
 
+// Entropy, mode selection and per-head attention (bc_entropy_dispatch_attention):
+// (out, modes uint8 [batch, n_heads]).
+std::tuple<torch::Tensor, torch::Tensor> entropy_dispatch_attention(
+    torch::Tensor Q, torch::Tensor K_bin, torch::Tensor K_res, torch::Tensor V_bin,
+    torch::Tensor V_res, int64_t batch, int64_t n_heads, int64_t n_kv_heads, int64_t seq_len,
+    int64_t kv_stride, int64_t head_dim, double threshold) {
+    check_q(Q, batch, n_heads, head_dim);
+    check_heads(n_heads, n_kv_heads, seq_len, kv_stride);
+    const CachePtrs c = cache_blobs(Q, K_bin, K_res, V_bin, V_res, batch * n_kv_heads * kv_stride);
+    c10::DeviceGuard guard(Q.device());
+    size_t ws_bytes = 0;
+    check_status(bc_entropy_dispatch_workspace_size((int)batch, (int)n_heads, (int)n_kv_heads,
+                                                    (int)seq_len, (int)head_dim, &ws_bytes),
+                 "entropy_dispatch_workspace_size");
+    auto ws = workspace_for(Q, ws_bytes);
+    auto out = torch::empty({batch, n_heads, head_dim}, Q.options());
+    auto modes = torch::empty({batch, n_heads}, Q.options().dtype(torch::kUInt8));
+    check_status(bc_entropy_dispatch_attention(Q.data_ptr(), c.kb, c.kr, c.vb, c.vr,
+                                               modes.data_ptr<uint8_t>(), out.data_ptr(), (int)batch,
+                                               (int)n_heads, (int)n_kv_heads, (int)seq_len,
+                                               (int)kv_stride, (int)head_dim, (float)threshold,
+                                               ws.data_ptr(), ws_bytes, stream_of(Q)),
+                 "entropy_dispatch_attention");
+    return {out.view(Q.sizes()), modes};
+}
+
 // One decode step: append the token (k, v: [batch*n_kv_heads*head_dim] fp16) at
 // position current_len % max_seq of the ring caches, then attend over the
 // filled positions (bc_append_attention).
@@ -680,6 +706,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("attention", &attention, "GQA / ring-stride binary or compensated attention");
     m.def("append_attention", &append_attention, "One decode step: ring-cache append + attention");
     m.def("head_mode_attention", &head_mode_attention, "Per-head binary / compensated attention");
+    m.def("entropy_dispatch_attention", &entropy_dispatch_attention,
+          "Entropy, mode selection and per-head attention");
     m.def("attention_partial", &attention_partial, "Split-KV partials (phase 1 of attention)");
     m.def("attention_combine", &attention_combine, "Merge split-KV partials (phase 2)");
     m.def("adaptive_attention", &adaptive_attention, "Top-k residual selection attention");

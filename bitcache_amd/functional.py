@@ -146,17 +146,17 @@ def entropy_dispatch_attention(Q: Tensor, K_bin: Tensor, K_res: Tensor, V_bin: T
     """The reference's adaptive precision end to end: per-head entropy of the binary
     scores (src/adaptive_precision.cu:13-130), mode = binary where entropy >= threshold
     (:133-144), then head_mode_attention.  Returns (out, modes)."""
-    kw = dict(n_kv_heads=n_kv_heads, kv_stride=kv_stride)
-    ent = compute_head_entropy(Q, K_bin, batch, n_heads, seq_len, head_dim, **kw)
-    modes = adaptive_select(ent, threshold).view(batch, n_heads)
+    _require_extension()
+    _check_q(Q)
     hkv = n_heads if n_kv_heads is None else n_kv_heads
     if kv_stride is None:
-        # the stride compute_head_entropy read with: the blob's capacity per kv row
-        # (a prefix view of a ring reads the ring's own stride)
-        kv_stride = _capacity(K_bin, _C.sizeof_binary_vec()) // max(batch * hkv, 1)
-    out = head_mode_attention(Q, K_bin, K_res, V_bin, V_res, modes, batch, n_heads, seq_len,
-                              head_dim, n_kv_heads=hkv, kv_stride=kv_stride)
-    return out, modes
+        # the stride compute_head_entropy reads with: seq_len given n_kv_heads, else
+        # the blob's capacity per kv row (a prefix view of a ring reads the ring's
+        # own stride)
+        kv_stride = (seq_len if n_kv_heads is not None else
+                     _capacity(K_bin, _C.sizeof_binary_vec()) // max(batch * hkv, 1))
+    return _C.entropy_dispatch_attention(Q, K_bin, K_res, V_bin, V_res, batch, n_heads, hkv, seq_len,
+                                         kv_stride, head_dim, threshold)
 
 
 def _capacity(blob: Tensor, per: int) -> int:

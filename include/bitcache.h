@@ -226,12 +226,23 @@ int bc_attention_combine(const void* workspace, void* out, int batch, int n_head
  * bc_adaptive_select from bc_compute_head_entropy).  The reference's intent
  * for adaptive precision (src/adaptive_precision.cuh:6-49), which its demo
  * dispatches per layer in Python (examples/generation_demo.py:129-141).
- * head_dim a multiple of 32 up to 256 (the matrix-core kernel at 64, 128 and
- * 256, the VALU kernel otherwise); workspace as bc_attention_workspace_size. */
+ * head_dim a multiple of 32 up to 256; workspace as bc_attention_workspace_size. */
 int bc_head_mode_attention(const void* q, const void* k_bin, const void* k_res, const void* v_bin,
                            const void* v_res, const uint8_t* modes, void* out, int batch,
                            int n_heads, int n_kv_heads, int seq_len, int kv_stride, int head_dim,
                            void* workspace, size_t workspace_bytes, void* stream);
+
+/* The reference's adaptive precision end to end: the heads' entropies
+ * (bc_compute_head_entropy_ws), modes[b*n_heads + h] = entropy >= threshold ? 0 :
+ * 1 (bc_adaptive_select; written) and bc_head_mode_attention with them, the
+ * modes and the group lists formed in one launch. */
+int bc_entropy_dispatch_workspace_size(int batch, int n_heads, int n_kv_heads, int seq_len,
+                                       int head_dim, size_t* bytes);
+int bc_entropy_dispatch_attention(const void* q, const void* k_bin, const void* k_res,
+                                  const void* v_bin, const void* v_res, uint8_t* modes, void* out,
+                                  int batch, int n_heads, int n_kv_heads, int seq_len, int kv_stride,
+                                  int head_dim, float threshold, void* workspace,
+                                  size_t workspace_bytes, void* stream);
 
 /* One decode step on ring caches of capacity batch*n_kv_heads*max_seq: the new
  * token k_new / v_new ([batch*n_kv_heads, head_dim] fp16) is encoded into

@@ -633,3 +633,27 @@ def test_entropy_dispatch_attention(F):
     for b in range(B):
         for h in range(H):
             close(out[b, h], rc[b, h] if modes[b, h] else rb[b, h], what=f"head ({b}, {h})")
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,stride,d", [(1, 4, 4, 1, 1, 128), (2, 8, 2, 700, 703, 96), (2, 8, 8, 9001, 9001, 64),
+                                                 (1, 1200, 300, 130, 140, 32), (1, 16, 8, 20000, 20001, 256)])
+def test_entropy_dispatch_equals_its_three_calls(F, B, Hq, Hkv, S, stride, d):
+    """entropy_dispatch_attention (entropies, modes and group lists in one
+    launch after the entropy pass) gives the modes and output, bit for bit, of
+    compute_head_entropy, adaptive_select and head_mode_attention: one and
+    several key chunks per head, GQA and ring strides, more heads than the list
+    kernel has threads, thresholds that split the heads and that do not."""
+    say(f"case entropy dispatch {(B, Hq, Hkv, S, stride, d)}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(S + d)
+    q = torch.randn((B, Hq, d), generator=g, device="cuda")
+    q = (q * torch.where(torch.rand((B, Hq, 1), generator=g, device="cuda") < 0.5, 1.0, 0.1)).half()
+    enc = [F.encode_fused(torch.randn((B * Hkv * stride, d), generator=g, device="cuda").half()) for _ in range(2)]
+    (kb, kr), (vb, vr) = enc
+    kw = dict(n_kv_heads=Hkv, kv_stride=stride)
+    ent = F.compute_head_entropy(q, kb, B, Hq, S, d, **kw)
+    for thr in (float(ent.median()), -1.0, 1e9):
+        modes = F.adaptive_select(ent, thr).view(B, Hq)
+        want = F.head_mode_attention(q, kb, kr, vb, vr, modes, B, Hq, S, d, **kw)
+        out, got = F.entropy_dispatch_attention(q, kb, kr, vb, vr, B, Hq, S, d, thr, **kw)
+        assert torch.equal(got, modes) and torch.equal(out, want), f"threshold {thr}"
