@@ -217,8 +217,8 @@ class BitCache:
     # ------------------------------------------------------------------ helpers
     def _validate_kv(self, K: Tensor, V: Tensor) -> None:
         expected = (self.batch, self.n_kv_heads, self.head_dim)
-        assert K.shape == torch.Size(expected), f"K shape {tuple(K.shape)} != {expected}"
-        assert V.shape == torch.Size(expected), f"V shape {tuple(V.shape)} != {expected}"
+        assert K.shape == expected, f"K shape {tuple(K.shape)} != {expected}"
+        assert V.shape == expected, f"V shape {tuple(V.shape)} != {expected}"
         assert K.dtype == torch.float16, "K must be float16"
         assert V.dtype == torch.float16, "V must be float16"
         assert K.is_cuda and V.is_cuda, "K and V must be on a ROCm device"

@@ -1073,14 +1073,29 @@ size_t list_bytes(int64_t groups) { return kListHeader + 2 * (size_t)groups * si
 
 // workspace of the split partials: the largest plan of any policy
 // plan_per_cu can return (per_cu = 0 .. kPlanMha), and the group lists
+//
+// One call asks for it up to three times (the workspace query, an entry
+// point's check, the launch's) with the same arguments, so each thread keeps
+// its last answer, a function of these integers alone.
 size_t ws_bytes(int batch, int hq, int hkv, int S, int D, int cu = 0) {
+    struct Last {
+        int batch, hq, hkv, S, D, cu;
+        size_t bytes;
+    };
+    static thread_local Last last = {-1, 0, 0, 0, 0, 0, 0};
+    if (cu <= 0) cu = bc::device_cu_count();
+    if (last.batch == batch && last.hq == hq && last.hkv == hkv && last.S == S && last.D == D &&
+        last.cu == cu)
+        return last.bytes;
     size_t n = plan_bytes(batch, hq, plan_splits(batch, hq, hkv, S, 0, cu), D);
     for (int per_cu = 1; per_cu <= kPlanMha; per_cu++) {
         const size_t b = plan_bytes(batch, hq, plan_splits(batch, hq, hkv, S, per_cu, cu), D);
         n = b > n ? b : n;
     }
     const int G = pick_g(hq / hkv);
-    return list_offset(n) + list_bytes((int64_t)batch * hkv * ((hq / hkv) / G));
+    n = list_offset(n) + list_bytes((int64_t)batch * hkv * ((hq / hkv) / G));
+    last = Last{batch, hq, hkv, S, D, cu, n};
+    return n;
 }
 
 int validate_heads(int batch, int n_heads, int n_kv_heads, int seq_len, int kv_stride, int d) {
