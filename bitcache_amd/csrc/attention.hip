@@ -937,8 +937,10 @@ SplitPlan plan_splits(int batch, int hq, int hkv, int S, int per_cu, int cu = 0)
     if (max_split > kMaxSplits) max_split = kMaxSplits;   // the combine kernel's weight table
     if (max_split < 1) max_split = 1;
     // ... and one per wave while every workgroup has a CU to itself (32/8
-    // heads of 4096 keys: 8 splits 12.9 us, 16 splits 11.8)
-    if (groups > 0 && groups * max_split < cu) {
+    // heads of 4096 keys: 8 splits 12.9 us, 16 splits 11.8), but for one split,
+    // which needs no merge launch (2x32 binary heads of 579 keys, d = 64: 7.9 us,
+    // two splits 11.0)
+    if (groups > 0 && max_split > 1 && groups * max_split < cu) {
         const int64_t alone = cu / groups < tiles / 4 ? cu / groups : tiles / 4;
         if (alone > max_split) max_split = alone < kMaxSplits ? (int)alone : kMaxSplits;
     }
@@ -1210,10 +1212,10 @@ int run_partial(int mode, const void* q, const void* k_bin, const void* k_res, c
         a.app_slot = app->slot;
     }
     const dim3 grid(p.n_splits, batch * n_kv_heads * ((n_heads / n_kv_heads) / p.G));
-    // matrix-core value phase for head_dim 64/128/256; the VALU kernel covers the
-    // other head dims (and is selectable with BITCACHE_VALU_ATTENTION=1).  With
-    // one split per group the matrix-core kernel normalises and writes the
-    // output itself (no merge launch).
+    // the matrix-core kernel, but for splits past its offsets' range (the VALU
+    // kernel, selectable with BITCACHE_VALU_ATTENTION=1).  With one split per
+    // group the matrix-core kernel normalises and writes the output itself (no
+    // merge launch).
     if (direct_out != nullptr && p.n_splits == 1) a.out = (uint16_t*)direct_out;
     // Per-head modes: the groups whose heads are all binary go to the binary
     // kernel, which reads none of their residual bytes, the others to the

@@ -1,10 +1,10 @@
-// One vector of the row encoder, shared by the encode kernels (encode.hip) and
-// the attention kernel's in-place append (attention_mfma.hip).
+// One vector of the one-slice row encoder: the attention kernel's in-place
+// append (attn_mfma_kernel.h) encodes a token's K and V with it.
 //
 // d in {64, 128, 256}: L = d/8 lanes per vector, lane j (0 <= j < L) of its
 // L-lane group holding elements 8j..8j+7 (one 16-byte load); a wave holds
 // 64/L such groups, lane = group * L + j, and every lane of the wave calls
-// encode_row (the reductions are DPP / swizzle moves within the group).  The
+// encode_row_slice (the reductions are DPP / swizzle moves within the group).  The
 // scale sum follows the reference tree exactly: element t = 8j + k sits in
 // lane j, so the tree levels s = 64..8 (src/binary_encode.cu:44-50) pair lane
 // j with lane j + s/8 (row_shl) and the levels s = 4, 2, 1 are in-lane; d = 256
@@ -169,12 +169,6 @@ __device__ __forceinline__ void encode_row_slice(const bc_v4u raw, int j, bool l
             if (j == 0) dst.rscale_plane[dv] = f2h(absmax);
         }
     }
-}
-
-template <int D, int MODE>
-__device__ __forceinline__ void encode_row(const uint16_t* vec, int j, bool live, const EncodeDst& dst,
-                                           int64_t dv) {
-    encode_row_slice<D, MODE>(load_row_slice(vec, j), j, live, dst, dv);
 }
 
 }  // namespace bc
