@@ -1296,33 +1296,35 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
         // redone (one wave max) only when a key exceeds it, and then only lowered
         float wfac = 1.0f;   // (int8 path) the factor that lowering applies
         {
-            const float wb = valid ? fmaxf(2.0f * svv, rsv * (1.0f / 7.0f)) : 0.0f;
+            // (a scale that is not finite takes no part: the heads that read it are
+            // NaN whatever the plan, a head that reads only the key's other part
+            // needs its weights planned all the same)
+            const float wa = 2.0f * svv, wr = rsv * (1.0f / 7.0f);
+            const float wb = valid ? fmaxf(wa < INFINITY ? wa : 0.0f, wr < INFINITY ? wr : 0.0f) : 0.0f;
             if (__ballot(wb > wlim) != 0ull) {
                 const float wmx = wave_max(wb);
-                if (wmx < INFINITY) {
-                    const int e = kWTop - kTauI - kSlack - (int)ceilf(log2f(wmx));
-                    if (have_wexp) {
-                        // a larger weight than planned (e < wexp): bring the sums down
-                        const float f = ldexpf(1.0f, e - wexp);
-                        if constexpr (I8) {
-                            wfac = f;   // applied by the flush below
-                        } else {
+                const int e = kWTop - kTauI - kSlack - (int)ceilf(log2f(wmx));
+                if (have_wexp) {
+                    // a larger weight than planned (e < wexp): bring the sums down
+                    const float f = ldexpf(1.0f, e - wexp);
+                    if constexpr (I8) {
+                        wfac = f;   // applied by the flush below
+                    } else {
 #pragma unroll
-                            for (int h = 0; h < NH; h++)
+                        for (int h = 0; h < NH; h++)
 #pragma unroll
-                                for (int p = 0; p < 4; p++) cs[h][p] *= f;
-                        }
-                        if constexpr (!R8) {
-#pragma unroll
-                            for (int d = 0; d < NB; d++) cn[d] *= f;
-                        }
-#pragma unroll
-                        for (int g = 0; g < G; g++) off[g] *= f;
+                            for (int p = 0; p < 4; p++) cs[h][p] *= f;
                     }
-                    wexp = e;
-                    have_wexp = true;
-                    wlim = ldexpf(1.0f, kWTop - kTauI - wexp);
+                    if constexpr (!R8) {
+#pragma unroll
+                        for (int d = 0; d < NB; d++) cn[d] *= f;
+                    }
+#pragma unroll
+                    for (int g = 0; g < G; g++) off[g] *= f;
                 }
+                wexp = e;
+                have_wexp = true;
+                wlim = ldexpf(1.0f, kWTop - kTauI - wexp);
             }
         }
 
