@@ -1341,10 +1341,11 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
         // weight b = p * fb, and the offset sum_s (a_s + 8 b_s) grows by p * fo
         const float fa = ldexpf(2.0f * svv * kfac, wexp);
         const float fb = RES ? ldexpf(rsv * (1.0f / 7.0f) * kfac_res, wexp) : 0.0f;
-        const float fo_bin = ldexpf(svv, wexp);
-        // (int8 codes need no offset; a V scale that is not finite has no
-        // integer weight, and makes the offset, so the output, NaN)
-        const float fo_res = R8 ? fmaf(svv + rsv, 0.0f, fo_bin) : RES ? ldexpf(svv + rsv * (8.0f / 7.0f), wexp) : fo_bin;
+        // (int8 path: a V scale that is not finite has no integer weight, and
+        // makes the offset, so the output of the heads that read it, NaN, as
+        // the sums of the fp16 path are; its codes need no offset)
+        const float fo_bin = I8 ? fmaf(svv, 0.0f, ldexpf(svv, wexp)) : ldexpf(svv, wexp);
+        const float fo_res = R8 ? fmaf(rsv, 0.0f, fo_bin) : RES ? ldexpf(svv + rsv * (8.0f / 7.0f), wexp) : fo_bin;
         // residual weights go to the slot of the key's residual position
         // (adaptive: compacted; unselected keys write zeros to the positions
         // past nsel, so every slot a residual MFMA reads is written)

@@ -106,6 +106,27 @@ def rel_error(mode, shape, gap, outliers):
 BAR = 2.0 ** -10
 
 
+@pytest.mark.parametrize("mode", ["binary", "compensated", "adaptive", "mixed"])
+@pytest.mark.parametrize("G", [1, 2, 4, 8])
+def test_value_scale_not_finite(mode, G):
+    """A V row whose scale is infinite or NaN (what an infinite element
+    encodes to): no sum of the heads that read it is a number, in any mode and
+    whatever the row's sign bits; the other kv head's are as without it."""
+    from bitcache_amd import functional as F, layout
+    B, Hkv, S, d = 1, 2, 500, 128
+    Hq = Hkv * G
+    q, blobs, _ = make(B, Hq, Hkv, S, d, 1.0, 1, seed=G)
+    clean, _ = attend(mode, q, blobs, B, Hq, Hkv, S, d)
+    for bad in (math.inf, math.nan):
+        for key in (0, 70, 499):
+            say(f"case V scale {bad} at key {key}, {mode}, group {G}")
+            vb = blobs[2].clone()
+            layout.binary_planes(vb, d)[1][key] = bad
+            out, _ = attend(mode, q, blobs[:2] + [vb] + blobs[3:], B, Hq, Hkv, S, d)
+            assert torch.isnan(out[0, :G]).all()
+            assert torch.equal(out[0, G:], clean[0, G:])
+
+
 @pytest.mark.parametrize("G", [1, 2, 4, 8])
 def test_residual_scale_not_finite(G):
     """A V residual scale that is infinite or NaN: the compensated heads that
