@@ -1341,20 +1341,22 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
         // weight b = p * fb, and the offset sum_s (a_s + 8 b_s) grows by p * fo
         const float fa = ldexpf(2.0f * svv * kfac, wexp);
         const float fb = RES ? ldexpf(rsv * (1.0f / 7.0f) * kfac_res, wexp) : 0.0f;
+        const float fo_bin = ldexpf(svv, wexp);
+        const float fo_res = RES ? ldexpf(svv + rsv * (8.0f / 7.0f), wexp) : fo_bin;
         // (int8 path: a V scale that is not finite has no integer weight, and
         // makes the offset, so the output of the heads that read it, NaN, as
-        // the sums of the fp16 path are; its codes need no offset)
-        const float fo_bin = I8 ? fmaf(svv, 0.0f, ldexpf(svv, wexp)) : ldexpf(svv, wexp);
-        const float fo_res = R8 ? fmaf(rsv, 0.0f, fo_bin) : RES ? ldexpf(svv + rsv * (8.0f / 7.0f), wexp) : fo_bin;
+        // the sums of the fp16 path are)
+        const float nan_bin = svv * 0.0f, nan_res = fmaf(rsv, 0.0f, nan_bin);
         // residual weights go to the slot of the key's residual position
         // (adaptive: compacted; unselected keys write zeros to the positions
         // past nsel, so every slot a residual MFMA reads is written)
         uint16_t* wres = wsl;
         uint8_t* w8res = w8st;
         uint32_t dsig[G], dres[G];   // (int8 path) packed digits
-        // the weight p * f <= 2^30, rounded (weights are not negative), as
+        // the weight p * f <= 2^30, rounded (weights are not negative), and its
         // balanced digits
-        auto pack8 = [](float p, float f) { return ((uint32_t)(int)fmaf(p, f, 0.5f) + 0x80808080u) ^ 0x80808080u; };
+        auto round8 = [](float p, float f) { return (uint32_t)(int)fmaf(p, f, 0.5f); };
+        auto pack8 = [](uint32_t w) { return (w + 0x80808080u) ^ 0x80808080u; };
         if constexpr (MODE == MODE_ADAPTIVE && I8)
             w8res = &lds_w8[0][0] + opaque_int((wave * 64 + slot8_of(res_row(rpos))) * kWRow);
         else if constexpr (MODE == MODE_ADAPTIVE)
@@ -1379,21 +1381,25 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
             if constexpr (MODE == MODE_MIXED) with_res = hmode[g];
             if constexpr (MODE == MODE_ADAPTIVE) with_res = (selmask >> g) & 1u;
             const float bv = with_res ? p * fb : 0.0f;
-            const float fo = with_res ? fo_res : fo_bin;
-            // offset removed at the end, from the unrounded weights: the (hi, lo)
-            // pairs carry ~22 bits (int8 path: rounding to integers up to
-            // 2^30), so the difference is a zero-mean term below 2^-22
-            off[g] = fmaf(p, fo, off[g]);
+            // the offset a = a2 / 2 of each key, taken off at the end.  int8
+            // path: half the rounded weight, so that the key's sum stays +-a of
+            // one a (half the unrounded one moves every dimension of the head
+            // the same way, by the rounding errors of all keys: one key 15.5
+            // nats above 65536 others, 1.7e-3 of the output).  fp16 path: the
+            // (hi, lo) pairs carry ~22 bits, a zero-mean difference
             if constexpr (I8) {
-                dsig[g] = pack8(p, fa);
+                const uint32_t w = round8(p, fa);
+                off[g] = fmaf(0.5f, (float)w, off[g]) + (with_res ? nan_res : nan_bin);
+                dsig[g] = pack8(w);
             } else {
+                off[g] = fmaf(p, with_res ? fo_res : fo_bin, off[g]);
                 const uint16_t a2h = f2h_bits(a2);
                 const uint16_t a2l = f2h_bits(a2 - h_bits2f(a2h));
                 wsl[(0 * 2 * G + 2 * g) * WL::kColSlots] = a2h;
                 wsl[(0 * 2 * G + 2 * g + 1) * WL::kColSlots] = a2l;
             }
             if constexpr (R8) {
-                dres[g] = pack8(p, with_res ? fb : 0.0f);
+                dres[g] = pack8(round8(p, with_res ? fb : 0.0f));
             } else if constexpr (RES) {
                 const uint16_t bh = f2h_bits(bv);
                 const uint16_t bl = f2h_bits(bv - h_bits2f(bh));

@@ -105,6 +105,22 @@ def rel_error(mode, shape, gap, outliers):
 # 2^-11 nats, which moves a weight by as much
 BAR = 2.0 ** -10
 
+# (mode, (B, Hq, Hkv, S, d)): plans of one split of 16K keys per wave
+LONG = [("binary", (8, 32, 32, 131072, 64)),
+        ("compensated", (32, 32, 8, 65536, 256)),
+        ("adaptive", (32, 8, 8, 65536, 160))]
+
+
+@pytest.mark.parametrize("mode,shape", LONG, ids=lambda x: str(x))
+def test_one_key_above_a_long_tail(mode, shape):
+    """A tail each of whose weights is near or below the resolution of the
+    integer weights: together it is a visible share of the softmax sum."""
+    for gap in (12.0, 13.5, 14.5, 15.5):
+        err = rel_error(mode, shape, gap, 1)
+        say(f"case one key {mode} {shape} gap {gap}: error {err:.2e}")
+        assert err <= BAR
+    torch.cuda.empty_cache()
+
 
 @pytest.mark.parametrize("mode", ["binary", "compensated", "adaptive", "mixed"])
 @pytest.mark.parametrize("G", [1, 2, 4, 8])
