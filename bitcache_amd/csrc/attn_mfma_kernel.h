@@ -192,6 +192,11 @@ __device__ __forceinline__ float xnor_score(float scale_q, float scale_k, float 
     return (scale_q * scale_k) * mq;
 }
 
+// 1 / f of a power of two between 2^-126 and 2^126
+__device__ __forceinline__ float pow2_inv(float f) {
+    return __builtin_bit_cast(float, 0x7F000000u - __builtin_bit_cast(uint32_t, f));
+}
+
 // a wave-uniform float, in a scalar register
 __device__ __forceinline__ float uniform_f(float f) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f)));
@@ -522,7 +527,7 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
     // to 2^30 in four balanced 8-bit digit columns (columns 4g + j): the bytes
     // of w + 0x80808080, each less 128, so two operations give the packed
     // word.  The sums are exact in int32 accumulators.  A rescale (running max
-    // or weight plan) flushes them, scaled, into a per-wave float bank in LDS
+    // or weight scale) flushes them, scaled, into a per-wave float bank in LDS
     // and restarts them at zero (flush8).
     // R8: the residual part too.  A code n enters as 16 n, eight codes in three
     // operations, its weight as digits of the same kind, and no offset is
@@ -557,7 +562,7 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
     __shared__ __attribute__((aligned(16))) int lds_rd[NW][WL::kRdInts];
     __shared__ __attribute__((aligned(16))) int lds_rdlo[NW][(KMF && G > 1 && 3 * G <= 16) ? WL::kRdInts : 1];
     __shared__ float wofs[NW][G];
-    __shared__ float wm[NW][G], wlsum[NW][G], wsc[NW];
+    __shared__ float wm[NW][G], wlsum[NW][G], wsc[NW][G];
 
     const int split = blockIdx.x;
     // per-head modes: this launch's query-head groups come from its list
@@ -946,17 +951,36 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
         live8 = 0;
     };
 
-    // weights enter the MFMAs as w * 2^wexp (fp16 hi + lo), wexp chosen so the
-    // largest possible weight sits near 2^14 (int8 path: integers up to 2^30):
-    // no overflow, and weights down to ~2^-30 of the largest keep their
-    // contribution (fp16; undone exactly in the epilogue).  The int8 path
-    // plans for value scales twice the largest seen, since lowering its plan
-    // costs a flush.
-    constexpr int kWTop = I8 ? 30 : 14;
-    constexpr int kSlack = I8 ? 1 : 0;
+    // fp16 path: weights enter the MFMAs as w * 2^wexp (hi + lo), wexp chosen so
+    // the largest possible weight sits near 2^14: no overflow, and weights down
+    // to ~2^-30 of the largest keep their contribution (undone exactly in the
+    // epilogue)
+    constexpr int kWTop = 14;
     int wexp = 0;
     bool have_wexp = false;
     float wlim = 0.0f;
+    // int8 path: weights enter as integers round(p f es), es a power of two per
+    // head.  es is planned from the weights themselves, not from the largest V
+    // scale a key may have: the integer step is then 2^-24 to 2^-31 of the
+    // largest weighted value since the head's last plan, whatever the rows that
+    // carry no weight are (a plan for the largest scale: one key 12 nats above
+    // 65536 others, one V row in 256 of 32 times the magnitude: 6.5e-3 of the
+    // output, planned from the weights 2e-4).  A weight past kW8Max, whose
+    // digits no longer fit, replans its head, and so does a move of the head's
+    // reference (which flushes the sums anyway): the tile's largest weight to
+    // [2^24, 2^25), so that it may grow 64 times before the next flush.  A flush
+    // waits for the loads in flight; scores of unit variance grow 8 times past
+    // a wave's first tile in 10 to 19% of the waves (d = 64, 96, 256: +8% of the
+    // kernel's time with 2^28 here), 64 times in less than 1%.  The step is far
+    // below the rounding of the fp16 output (2.1e-4): weights to 2^24, 2e-5 of
+    // it with one key 9 to 16 nats above 32768 others.
+    // Without any weight es stays at 2^60, below the last bit of any output.
+    constexpr float kW8Max = 2139000000.0f;   // <= 0x7F7F7F7F
+    constexpr int kW8Top = 25;
+    constexpr float kEsMax = 1152921504606846976.0f;   // 2^60
+    float es[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) es[g] = kEsMax;
 
     uint32_t thresh[G];
     int cutoff[G];
@@ -1291,11 +1315,10 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
             sc[g] = valid ? score * isd2 : -INFINITY;
         }
 
-        // weight scale: weights are p * wb * 2^wexp with p <= 2^kTau, so the
-        // plan holds while every wb <= wlim = 2^(kWTop - kTau - wexp); it is
+        // (fp16 path) weight scale: weights are p * wb * 2^wexp with p <= 2^kTau,
+        // so the plan holds while every wb <= wlim = 2^(kWTop - kTau - wexp); it is
         // redone (one wave max) only when a key exceeds it, and then only lowered
-        float wfac = 1.0f;   // (int8 path) the factor that lowering applies
-        {
+        if constexpr (!I8) {
             // (a scale that is not finite takes no part: the heads that read it are
             // NaN whatever the plan, a head that reads only the key's other part
             // needs its weights planned all the same)
@@ -1303,22 +1326,16 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
             const float wb = valid ? fmaxf(wa < INFINITY ? wa : 0.0f, wr < INFINITY ? wr : 0.0f) : 0.0f;
             if (__ballot(wb > wlim) != 0ull) {
                 const float wmx = wave_max(wb);
-                const int e = kWTop - kTauI - kSlack - (int)ceilf(log2f(wmx));
+                const int e = kWTop - kTauI - (int)ceilf(log2f(wmx));
                 if (have_wexp) {
                     // a larger weight than planned (e < wexp): bring the sums down
                     const float f = ldexpf(1.0f, e - wexp);
-                    if constexpr (I8) {
-                        wfac = f;   // applied by the flush below
-                    } else {
 #pragma unroll
-                        for (int h = 0; h < NH; h++)
+                    for (int h = 0; h < (I8 ? 0 : NH); h++)
 #pragma unroll
-                            for (int p = 0; p < 4; p++) cs[h][p] *= f;
-                    }
-                    if constexpr (!R8) {
+                        for (int p = 0; p < 4; p++) cs[h][p] *= f;
 #pragma unroll
-                        for (int d = 0; d < NB; d++) cn[d] *= f;
-                    }
+                    for (int d = 0; d < (I8 ? 0 : NB); d++) cn[d] *= f;
 #pragma unroll
                     for (int g = 0; g < G; g++) off[g] *= f;
                 }
@@ -1328,39 +1345,41 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
             }
         }
 
-        // online softmax; (hi, lo) fp16 weights to LDS in MFMA slot order
-        float lane_alpha = 1.0f;
+        // online softmax; (hi, lo) fp16 weights, or the digits of the integer
+        // weights, to LDS in MFMA slot order
+        float lane_alpha = 1.0f;   // the factor of the lane's head's sums so far
         bool any_rescale = false;
         // the value operands of odd rows come out 16x larger (see the MFMA
         // loops below): their weights carry 1/16 so that every product is exact
         // (the residual row of a key is its compacted position's row, of the
-        // parity of rpos); the int8 sign elements carry no such factor
+        // parity of rpos); the int8 elements carry no such factor
         const float kfac = (!I8 && (kown & 1)) ? 0.0625f : 1.0f;
-        const float kfac_res = (!R8 && (rpos & 1)) ? 0.0625f : 1.0f;
+        const float kfac_res = (!I8 && (rpos & 1)) ? 0.0625f : 1.0f;
         // per-key factors shared by the heads: sign weight a2 = p * fa, residual
-        // weight b = p * fb, and the offset sum_s (a_s + 8 b_s) grows by p * fo
-        const float fa = ldexpf(2.0f * svv * kfac, wexp);
-        const float fb = RES ? ldexpf(rsv * (1.0f / 7.0f) * kfac_res, wexp) : 0.0f;
-        const float fo_bin = ldexpf(svv, wexp);
-        const float fo_res = RES ? ldexpf(svv + rsv * (8.0f / 7.0f), wexp) : fo_bin;
-        // (int8 path: a V scale that is not finite has no integer weight, and
-        // makes the offset, so the output of the heads that read it, NaN, as
-        // the sums of the fp16 path are)
-        const float nan_bin = svv * 0.0f, nan_res = fmaf(rsv, 0.0f, nan_bin);
+        // weight b = p * fb; (fp16) the offset sum_s (a_s + 8 b_s) grows by p * fo
+        const float fa = I8 ? 2.0f * svv : ldexpf(2.0f * svv * kfac, wexp);
+        const float fb = !RES ? 0.0f : I8 ? rsv * (1.0f / 7.0f) : ldexpf(rsv * (1.0f / 7.0f) * kfac_res, wexp);
+        const float fo_bin = I8 ? 0.0f : ldexpf(svv, wexp);
+        const float fo_res = (RES && !I8) ? ldexpf(svv + rsv * (8.0f / 7.0f), wexp) : fo_bin;
         // residual weights go to the slot of the key's residual position
         // (adaptive: compacted; unselected keys write zeros to the positions
         // past nsel, so every slot a residual MFMA reads is written)
         uint16_t* wres = wsl;
         uint8_t* w8res = w8st;
-        uint32_t dsig[G], dres[G];   // (int8 path) packed digits
-        // the weight p * f <= 2^30, rounded (weights are not negative), and its
-        // balanced digits
-        auto round8 = [](float p, float f) { return (uint32_t)(int)fmaf(p, f, 0.5f); };
-        auto pack8 = [](uint32_t w) { return (w + 0x80808080u) ^ 0x80808080u; };
         if constexpr (MODE == MODE_ADAPTIVE && I8)
             w8res = &lds_w8[0][0] + opaque_int((wave * 64 + slot8_of(res_row(rpos))) * kWRow);
         else if constexpr (MODE == MODE_ADAPTIVE)
             wres = &lds_wts[0][0] + opaque_int(wave * (WL::kWeightBytes / 2) + slot_of(res_row(rpos)));
+        // does head g take the key's residual
+        auto with_res = [&](int g) {
+            if constexpr (MODE == MODE_MIXED) return hmode[g];
+            if constexpr (MODE == MODE_ADAPTIVE) return (bool)((selmask >> g) & 1u);
+            return MODE == MODE_COMP;
+        };
+        // (int8 path) p es per head, its sign and residual weights plus 1/2, and
+        // the heads whose reference moved
+        float ps[G], wsig[G], wresid[G], wtop = 0.0f;
+        uint32_t moved = 0u;
 #pragma unroll
         for (int g = 0; g < G; g++) {
             // the reference m[g] moves only when a score passes m[g] + kTau
@@ -1371,40 +1390,88 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
                 off[g] *= alpha;
                 if (my_head == g) lane_alpha = alpha;
                 any_rescale = true;
+                moved |= 1u << g;
                 m[g] = mn;
                 mlim[g] = mn + kTau;
             }
             const float p = valid ? __builtin_amdgcn_exp2f(sc[g] - m[g]) : 0.0f;
             lsum[g] += p;
-            const float a2 = p * fa;
-            bool with_res = MODE == MODE_COMP;   // the head takes the key's residual
-            if constexpr (MODE == MODE_MIXED) with_res = hmode[g];
-            if constexpr (MODE == MODE_ADAPTIVE) with_res = (selmask >> g) & 1u;
-            const float bv = with_res ? p * fb : 0.0f;
-            // the offset a = a2 / 2 of each key, taken off at the end.  int8
-            // path: half the rounded weight, so that the key's sum stays +-a of
-            // one a (half the unrounded one moves every dimension of the head
-            // the same way, by the rounding errors of all keys: one key 15.5
-            // nats above 65536 others, 1.7e-3 of the output).  fp16 path: the
-            // (hi, lo) pairs carry ~22 bits, a zero-mean difference
             if constexpr (I8) {
-                const uint32_t w = round8(p, fa);
-                off[g] = fmaf(0.5f, (float)w, off[g]) + (with_res ? nan_res : nan_bin);
-                dsig[g] = pack8(w);
+                ps[g] = p * es[g];
+                wsig[g] = fmaf(ps[g], fa, 0.5f);
+                wtop = fmaxf(wtop, wsig[g]);
+                if constexpr (RES) {
+                    wresid[g] = fmaf(ps[g], with_res(g) ? fb : 0.0f, 0.5f);
+                    wtop = fmaxf(wtop, wresid[g]);
+                }
             } else {
-                off[g] = fmaf(p, with_res ? fo_res : fo_bin, off[g]);
+                const float a2 = p * fa;
+                const float bv = with_res(g) ? p * fb : 0.0f;
+                // the offset a + 8 b of each key, taken off at the end: the (hi, lo)
+                // pairs carry ~22 bits, a zero-mean difference
+                off[g] = fmaf(p, with_res(g) ? fo_res : fo_bin, off[g]);
                 const uint16_t a2h = f2h_bits(a2);
                 const uint16_t a2l = f2h_bits(a2 - h_bits2f(a2h));
                 wsl[(0 * 2 * G + 2 * g) * WL::kColSlots] = a2h;
                 wsl[(0 * 2 * G + 2 * g + 1) * WL::kColSlots] = a2l;
+                if constexpr (RES) {
+                    const uint16_t bh = f2h_bits(bv);
+                    const uint16_t bl = f2h_bits(bv - h_bits2f(bh));
+                    wres[(kRes0 + 2 * g) * WL::kColSlots] = bh;
+                    wres[(kRes0 + 2 * g + 1) * WL::kColSlots] = bl;
+                }
             }
-            if constexpr (R8) {
-                dres[g] = pack8(round8(p, with_res ? fb : 0.0f));
-            } else if constexpr (RES) {
-                const uint16_t bh = f2h_bits(bv);
-                const uint16_t bl = f2h_bits(bv - h_bits2f(bh));
-                wres[(kRes0 + 2 * g) * WL::kColSlots] = bh;
-                wres[(kRes0 + 2 * g + 1) * WL::kColSlots] = bl;
+        }
+        uint32_t dsig[G], dres[G];   // (int8 path) packed digits
+        if constexpr (I8) {
+            if (moved != 0u || __ballot(wtop >= kW8Max) != 0ull) {
+                // (weights that are not finite take no part: their head is NaN,
+                // below, and the group's other heads do not have them)
+                uint32_t wmx[G];
+#pragma unroll
+                for (int g = 0; g < G; g++) {
+                    float w = wsig[g] < INFINITY ? wsig[g] : 0.0f;
+                    if constexpr (RES) w = fmaxf(w, wresid[g] < INFINITY ? wresid[g] : 0.0f);
+                    wmx[g] = __builtin_bit_cast(uint32_t, w);
+                }
+                wave_umax(wmx);
+#pragma unroll
+                for (int g = 0; g < G; g++) {
+                    if ((moved >> g & 1u) || wmx[g] >= __builtin_bit_cast(uint32_t, kW8Max)) {
+                        // the largest weight is in [2^(e - 1), 2^e), e = its exponent
+                        // field - 126; 2^kW8Top-e by its own exponent field
+                        const int e = (int)(wmx[g] >> 23) - 126;
+                        const float en = fminf(es[g] * __builtin_bit_cast(float, (uint32_t)(127 + kW8Top - e) << 23), kEsMax);
+                        const float f = uniform_f(en * pow2_inv(es[g]));
+                        es[g] = uniform_f(en);
+                        ps[g] *= f;
+                        off[g] *= f;
+                        wsig[g] = fmaf(ps[g], fa, 0.5f);
+                        if constexpr (RES) wresid[g] = fmaf(ps[g], with_res(g) ? fb : 0.0f, 0.5f);
+                        if (my_head == g) lane_alpha *= f;
+                        any_rescale = true;
+                    }
+                }
+            }
+            // a V scale that is not finite has no integer weight: it makes the
+            // offset, so the output of the heads that read it, NaN, as the sums
+            // of the fp16 path are
+            if (__ballot(!(svv + (RES ? rsv : 0.0f) < INFINITY)) != 0ull) {
+#pragma unroll
+                for (int g = 0; g < G; g++) off[g] += svv * 0.0f + (with_res(g) ? rsv * 0.0f : 0.0f);
+            }
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                // (weights are not negative: truncation after adding 1/2 rounds)
+                const uint32_t w = (uint32_t)(int)wsig[g];
+                // the offset a = a2 / 2 of each key, taken off at the end: half the
+                // rounded weight, so that the key's sum stays +-a of one a (half
+                // the unrounded one moves every dimension of the head the same
+                // way, by the rounding errors of all keys)
+                off[g] = fmaf(0.5f, (float)w, off[g]);
+                // balanced digits
+                dsig[g] = (w + 0x80808080u) ^ 0x80808080u;
+                if constexpr (RES) dres[g] = ((uint32_t)(int)wresid[g] + 0x80808080u) ^ 0x80808080u;
             }
         }
         if constexpr (I8 && G == 4) {
@@ -1427,10 +1494,9 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
         }
         if constexpr (I8) {
             // the integer sums so far move to the float bank, scaled by this
-            // tile's factors (rare: the weight plan was lowered, a score
-            // passed m + kTau, or the residual sums are full)
-            if (live8 > 0 && (any_rescale || wfac != 1.0f || (R8 && live8 >= kMaxTiles8)))
-                flush8(lane_alpha * wfac);
+            // tile's factors (rare: a score passed m + kTau, a weight kW8Max, or
+            // the residual sums are full)
+            if (live8 > 0 && (any_rescale || (R8 && live8 >= kMaxTiles8))) flush8(lane_alpha);
         } else if (any_rescale) {
             if (my_head >= G) lane_alpha = 1.0f;
 #pragma unroll
@@ -1699,9 +1765,9 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
             wm[wave][g] = m[g];
             wlsum[wave][g] = l_w;
             wofs[wave][g] = o_w;
+            wsc[wave][g] = I8 ? pow2_inv(es[g]) : ldexpf(1.0f, -wexp);
         }
     }
-    if (lane == 0) wsc[wave] = ldexpf(1.0f, -wexp);
     float* accw = (float*)lds_st0[wave];
     const float dscale = digit_scale();
     const float* const bank = bank_at();
@@ -1803,7 +1869,7 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
                 if (RES) v += aw[(1 * HP + hs2) * D + e];
                 const bool live = mw[w] != -INFINITY;
                 const float f = live ? __builtin_amdgcn_exp2f(mw[w] - M) : 0.0f;
-                accv += live && f != 0.0f ? (v * sunit - wofs[w][g]) * (f * wsc[w]) : 0.0f;
+                accv += live && f != 0.0f ? (v * sunit - wofs[w][g]) * (f * wsc[w][g]) : 0.0f;
                 if (live) L += f * wlsum[w][g];
             }
             if (a.out != nullptr) {

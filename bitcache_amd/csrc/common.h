@@ -115,6 +115,23 @@ __device__ __forceinline__ float wave_sum63(float v) {
     v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x143, 0xC, 0xF, false));
     return v;
 }
+// Max over the wave of each of N words, without LDS moves, as scalars (0 is the
+// identity: the bit patterns of floats that are not negative order as they do).
+template <int N>
+__device__ __forceinline__ void wave_umax(uint32_t (&v)[N]) {
+#define BC_UMAX_STEP(CTRL, ROWS)                                                                        \
+    _Pragma("unroll") for (int i = 0; i < N; i++)                                                       \
+        v[i] = max(v[i], (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[i], CTRL, ROWS, 0xF, false));
+    BC_UMAX_STEP(0x111, 0xF)   // row_shr 1, 2, 4, 8: a 16-lane row's max in its last lane
+    BC_UMAX_STEP(0x112, 0xF)
+    BC_UMAX_STEP(0x114, 0xF)
+    BC_UMAX_STEP(0x118, 0xF)
+    BC_UMAX_STEP(0x142, 0xA)   // row broadcasts into the rows after
+    BC_UMAX_STEP(0x143, 0xC)
+#undef BC_UMAX_STEP
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = (uint32_t)__builtin_amdgcn_readlane((int)v[i], 63);
+}
 __device__ __forceinline__ int lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
 
 // Sign-word loaders: D/8 bytes per vector, returned as D/32 uint32 words.

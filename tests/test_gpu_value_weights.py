@@ -167,3 +167,18 @@ def test_residual_scale_not_finite(G):
             assert err <= BAR, f"binary heads: error {err:.2e}"
             out, _ = attend("compensated", q, broken, B, Hq, Hkv, S, d)
             assert torch.isnan(out).all()
+
+
+@pytest.mark.parametrize("mode", ["binary", "compensated", "adaptive", "mixed"])
+@pytest.mark.parametrize("shape", [(1, 8, 8, 16384, 96), (1, 8, 2, 16384, 64), (2, 32, 8, 16384, 128),
+                                   (1, 16, 2, 16384, 128), (1, 4, 2, 9000, 256), (8, 32, 32, 65536, 128)],
+                         ids=lambda s: str(s))
+def test_rows_of_very_different_magnitude(mode, shape):
+    """One V row in 256 of 4 to 32 times the others' magnitude, with next to no
+    softmax weight: the resolution of the weights is that of the weighted
+    values, not of the largest row."""
+    for gap, outliers in ((9.0, 8), (9.0, 32), (12.0, 32), (14.0, 4)):
+        err = rel_error(mode, shape, gap, outliers)
+        say(f"case outlier rows {mode} {shape} gap {gap} x{outliers}: error {err:.2e}")
+        assert err <= BAR
+    torch.cuda.empty_cache()
