@@ -931,6 +931,10 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
                 }
             }
         if constexpr (R8) {
+            // (other lanes add to what the sign part's owners have stored)
+            __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             // (codes as 16 n)
 #pragma unroll
             for (int d = 0; d < NB; d++) {
