@@ -890,11 +890,25 @@ __global__ void select_kernel(const float* e, uint8_t* modes, int n, float thr) 
 }
 
 // ---------------------------------------------------------------- host side
-int pick_g(int group) {
-    if (group % 8 == 0) return 8;
+// Query heads per workgroup, of the `group` that share a kv head.
+int pick_g(int group, int most = 8) {
+    if (group % 8 == 0 && most >= 8) return 8;
     if (group % 4 == 0) return 4;
     if (group % 2 == 0) return 2;
     return 1;
+}
+
+// The same for an attention mode: at most four at d = 32, 96, 160, 192 and 224
+// but for adaptive attention, whose selection passes are laid out for eight.
+// The kernel's groups of eight sum fp16 products in fp32, which costs those head
+// dims accuracy that the fp32 kernel that ran them before, and two groups of
+// four on exact sums, have: 8x(64/8) heads of 9001 keys, unit variance, error
+// against 64 bits of the fp32 kernel / one group of eight / two of four: d = 32
+// 2.1e-4 / 2.5e-4 / 2.1e-4, d = 96 2.2 / 2.5 / 2.1, d = 192 2.4 / 2.6 / 2.2;
+// time: 82 / 22.9 / 21.0 us, 153 / 32.5 / 36.2, 315 / 56.0 / 58.9 (60000 keys,
+// d = 192, where the second reading of the keys counts: 1836 / 241 / 303).
+int attn_g(int group, int D, int mode) {
+    return pick_g(group, D == 64 || D == 128 || D == 256 || mode == MODE_ADAPTIVE ? 8 : 4);
 }
 
 struct SplitPlan {
@@ -927,9 +941,9 @@ struct SplitPlan {
 constexpr int kMaxPerCu = 4;
 constexpr int kPlanMha = kMaxPerCu + 1;
 constexpr int kShortTiles = 4;   // per wave
-SplitPlan plan_splits(int batch, int hq, int hkv, int S, int per_cu, int cu = 0) {
+SplitPlan plan_splits(int batch, int hq, int hkv, int S, int G, int per_cu, int cu = 0) {
     SplitPlan p;
-    p.G = pick_g(hq / hkv);
+    p.G = G;
     const int64_t groups = (int64_t)batch * hkv * ((hq / hkv) / p.G);
     const int tiles = (S + 63) / 64;
     if (cu <= 0) cu = bc::device_cu_count();
@@ -1089,12 +1103,14 @@ size_t ws_bytes(int batch, int hq, int hkv, int S, int D, int cu = 0) {
     if (last.batch == batch && last.hq == hq && last.hkv == hkv && last.S == S && last.D == D &&
         last.cu == cu)
         return last.bytes;
-    size_t n = plan_bytes(batch, hq, plan_splits(batch, hq, hkv, S, 0, cu), D);
-    for (int per_cu = 1; per_cu <= kPlanMha; per_cu++) {
-        const size_t b = plan_bytes(batch, hq, plan_splits(batch, hq, hkv, S, per_cu, cu), D);
-        n = b > n ? b : n;
-    }
-    const int G = pick_g(hq / hkv);
+    // (adaptive attention's groups may be larger than the other modes')
+    const int G = attn_g(hq / hkv, D, MODE_COMP), Ga = attn_g(hq / hkv, D, MODE_ADAPTIVE);
+    size_t n = 0;
+    for (int g = G; g <= Ga; g *= 2)
+        for (int per_cu = 0; per_cu <= kPlanMha; per_cu++) {
+            const size_t b = plan_bytes(batch, hq, plan_splits(batch, hq, hkv, S, g, per_cu, cu), D);
+            n = b > n ? b : n;
+        }
     n = list_offset(n) + list_bytes((int64_t)batch * hkv * ((hq / hkv) / G));
     last = Last{batch, hq, hkv, S, D, cu, n};
     return n;
@@ -1176,7 +1192,8 @@ int run_partial(int mode, const void* q, const void* k_bin, const void* k_res, c
     const size_t need_ws = ws_bytes(batch, n_heads, n_kv_heads, seq_len, head_dim);
     BC_REQUIRE(workspace != nullptr && workspace_bytes >= need_ws, BC_ERR_WORKSPACE,
                "workspace of %zu bytes required, got %zu", need_ws, workspace_bytes);
-    const SplitPlan p = plan_splits(batch, n_heads, n_kv_heads, seq_len, per_cu);
+    const SplitPlan p = plan_splits(batch, n_heads, n_kv_heads, seq_len,
+                                    attn_g(n_heads / n_kv_heads, head_dim, mode), per_cu);
     const int64_t groups = (int64_t)batch * n_kv_heads * ((n_heads / n_kv_heads) / p.G);
     // (the bound the launch needs: the partials of the plan it runs, and for
     // per-head modes the group lists after them)
@@ -1276,13 +1293,14 @@ int run_partial(int mode, const void* q, const void* k_bin, const void* k_res, c
     return bc::check_launch("attention split");
 }
 
-int run_combine(int per_cu, const void* workspace, void* out, int batch, int n_heads, int n_kv_heads,
+int run_combine(int mode, int per_cu, const void* workspace, void* out, int batch, int n_heads, int n_kv_heads,
                 int seq_len, int head_dim, hipStream_t st) {
     int v = validate_heads(batch, n_heads, n_kv_heads, seq_len, seq_len, head_dim);
     if (v != BC_OK) return v;
     if ((int64_t)batch * n_heads == 0) return BC_OK;
     BC_REQUIRE(workspace && out, BC_ERR_INVALID_ARGUMENT, "null pointer");
-    const SplitPlan p = plan_splits(batch, n_heads, n_kv_heads, seq_len, per_cu);
+    const SplitPlan p = plan_splits(batch, n_heads, n_kv_heads, seq_len,
+                                    attn_g(n_heads / n_kv_heads, head_dim, mode), per_cu);
     BC_DISPATCH_D(head_dim, launch_combine, (const float*)workspace, (uint16_t*)out,
                   batch * n_heads, p.n_splits, st);
     return bc::check_launch("attention combine");
@@ -1315,7 +1333,7 @@ static int run_attention_dispatch(int mode, const void* q, const void* k_bin, co
                                   const void* pcs, const AppendArgs* app, const uint8_t* head_mode,
                                   const DispatchArgs* dispatch) {
     const int per_cu = head_dim > 0 && n_kv_heads > 0
-                           ? plan_per_cu(mode, head_dim, pick_g(n_heads / n_kv_heads)) : kPlanFixed;
+                           ? plan_per_cu(mode, head_dim, attn_g(n_heads / n_kv_heads, head_dim, mode)) : kPlanFixed;
     BC_REQUIRE(out != nullptr || (int64_t)batch * n_heads == 0, BC_ERR_INVALID_ARGUMENT,
                "null output");
     bool wrote = false;
@@ -1323,7 +1341,7 @@ static int run_attention_dispatch(int mode, const void* q, const void* k_bin, co
                          kv_stride, head_dim, workspace, workspace_bytes, st, thresh, cutoff,
                          selected, pcs, per_cu, app, head_mode, out, &wrote, dispatch);
     if (rc != BC_OK || wrote) return rc;
-    return run_combine(per_cu, workspace, out, batch, n_heads, n_kv_heads, seq_len, head_dim, st);
+    return run_combine(mode, per_cu, workspace, out, batch, n_heads, n_kv_heads, seq_len, head_dim, st);
 }
 
 size_t attention_ws_bytes(int batch, int n_heads, int n_kv_heads, int seq_len, int d) {
@@ -1351,8 +1369,9 @@ extern "C" int bc_attention_split_plan(int mode, int batch, int n_heads, int n_k
     BC_REQUIRE(cu_count >= 0, BC_ERR_INVALID_ARGUMENT, "cu_count %d < 0", cu_count);
     BC_REQUIRE(n_splits && partial_bytes && workspace_bytes, BC_ERR_INVALID_ARGUMENT,
                "null output");
-    const int per_cu = plan_per_cu(mode, head_dim, pick_g(n_heads / n_kv_heads));
-    SplitPlan p = plan_splits(batch, n_heads, n_kv_heads, seq_len, per_cu, cu_count);
+    const int G = attn_g(n_heads / n_kv_heads, head_dim, mode);
+    const int per_cu = plan_per_cu(mode, head_dim, G);
+    SplitPlan p = plan_splits(batch, n_heads, n_kv_heads, seq_len, G, per_cu, cu_count);
     const int64_t groups = (int64_t)batch * n_kv_heads * ((n_heads / n_kv_heads) / p.G);
     if (wide_plan(mode, head_dim, p.G, groups, seq_len, cu_count > 0 ? cu_count : bc::device_cu_count())) {
         // (one wide workgroup per head; no partials are written)
@@ -1380,7 +1399,7 @@ extern "C" int bc_attention_partial(const void* q, const void* k_bin, const void
 extern "C" int bc_attention_combine(const void* workspace, void* out, int batch, int n_heads,
                                     int n_kv_heads, int seq_len, int head_dim, void* stream) {
     // (the partials of bc_attention_partial, planned with the same fixed policy)
-    return bc::run_combine(kPlanFixed, workspace, out, batch, n_heads, n_kv_heads, seq_len, head_dim,
+    return bc::run_combine(MODE_COMP, kPlanFixed, workspace, out, batch, n_heads, n_kv_heads, seq_len, head_dim,
                            (hipStream_t)stream);
 }
 
@@ -1491,10 +1510,10 @@ extern "C" int bc_append_attention(const void* q, const void* k_new, const void*
                "workspace of %zu bytes required, got %zu", need_ws, workspace_bytes);
     const int mode = k_res ? MODE_COMP : MODE_BINARY;
     const int group = n_heads / n_kv_heads;
-    const SplitPlan p = plan_splits(batch, n_heads, n_kv_heads, seq_len,
-                                    plan_per_cu(mode, head_dim, pick_g(group)));
+    const int G = attn_g(group, head_dim, mode);
+    const SplitPlan p = plan_splits(batch, n_heads, n_kv_heads, seq_len, G, plan_per_cu(mode, head_dim, G));
     hipStream_t st = (hipStream_t)stream;
-    if (valu_forced() || pick_g(group) != group || !bc::append_dim(head_dim) ||
+    if (valu_forced() || G != group || !bc::append_dim(head_dim) ||
         !bc::mfma_split_ok(head_dim, p.chunk)) {
         const int rc = bc_online_encode_kv(k_new, v_new, k_bin, k_res, v_bin, v_res, batch,
                                            n_kv_heads, head_dim, current_len, max_seq, stream);
@@ -1713,7 +1732,8 @@ extern "C" int bc_reference_attention(const void* q, const void* k, const void* 
     const size_t need_ws = ws_bytes(batch, n_heads, n_kv_heads, seq_len, head_dim);
     BC_REQUIRE(workspace != nullptr && workspace_bytes >= need_ws, BC_ERR_WORKSPACE,
                "workspace of %zu bytes required, got %zu", need_ws, workspace_bytes);
-    const SplitPlan p = plan_splits(batch, n_heads, n_kv_heads, seq_len, kPlanFixed);
+    const SplitPlan p = plan_splits(batch, n_heads, n_kv_heads, seq_len,
+                                    pick_g(n_heads / n_kv_heads), kPlanFixed);
     const dim3 grid(p.n_splits, batch * n_kv_heads * ((n_heads / n_kv_heads) / p.G));
     hipStream_t st = (hipStream_t)stream;
     BC_DISPATCH_D(head_dim, launch_ref, p.G, q, k, v, n_heads, n_kv_heads, seq_len, p.n_splits,

@@ -182,3 +182,26 @@ def test_rows_of_very_different_magnitude(mode, shape):
         say(f"case outlier rows {mode} {shape} gap {gap} x{outliers}: error {err:.2e}")
         assert err <= BAR
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("d", [32, 96, 160, 192, 224])
+@pytest.mark.parametrize("mode", ["binary", "compensated"])
+def test_groups_of_eight_at_every_head_dim(mode, d):
+    """Unit-variance heads of 9001 keys: what the kernel's sums add to the
+    rounding of the fp16 output is at most a quarter of that rounding (fp32 sums
+    of fp16 products with the codes' offset of 8 are past it)."""
+    from bitcache_amd import functional as F
+    B, Hkv, S, G = 1, 8, 9001, 8
+    g = torch.Generator(device="cuda")
+    g.manual_seed(d)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda").half()
+    q, k, v = rnd(B, Hkv * G, d), rnd(Hkv, S, d), rnd(Hkv, S, d)
+    kb, kr = F.encode_fused(k.view(-1, d))
+    vb, vr = F.encode_fused(v.view(-1, d))
+    out, with_res = attend(mode, q, (kb, kr, vb, vr), B, Hkv * G, Hkv, S, d)
+    want = torch.cat([exact(q[0, G * h:G * h + G], planes64(*F.encode_fused(k[h]), S, d),
+                            planes64(*F.encode_fused(v[h]), S, d), with_res) for h in range(Hkv)])
+    err = float((out[0].double() - want).norm() / want.norm())
+    rounding = float((want.half().double() - want).norm() / want.norm())
+    say(f"case groups of eight {mode} d={d}: error {err:.2e}, of rounding alone {rounding:.2e}")
+    assert err <= rounding * math.sqrt(1 + 0.25 ** 2)
