@@ -1001,6 +1001,13 @@ SplitPlan plan_splits(int batch, int hq, int hkv, int S, int G, int per_cu, int 
             const int64_t one_round = ((per_cu == kPlanMha ? 2LL : 3LL) * cu) / groups;
             want = one_round < max_split ? (int)one_round : max_split;
         }
+        // (groups of eight run as two of four: as many splits as one group of
+        // eight takes, so that the partials take no more room)
+        const int most = pick_g(hq / hkv);
+        if (G < most) {
+            const int n = plan_splits(batch, hq, hkv, S, most, per_cu, cu).n_splits;
+            if (want > n) want = n;
+        }
     }
     static const int forced = [] {
         const char* e = getenv("BITCACHE_SPLITS");
@@ -1103,14 +1110,21 @@ size_t ws_bytes(int batch, int hq, int hkv, int S, int D, int cu = 0) {
     if (last.batch == batch && last.hq == hq && last.hkv == hkv && last.S == S && last.D == D &&
         last.cu == cu)
         return last.bytes;
-    // (adaptive attention's groups may be larger than the other modes')
-    const int G = attn_g(hq / hkv, D, MODE_COMP), Ga = attn_g(hq / hkv, D, MODE_ADAPTIVE);
+    const int G = attn_g(hq / hkv, D, MODE_COMP), Gmax = pick_g(hq / hkv);
     size_t n = 0;
-    for (int g = G; g <= Ga; g *= 2)
-        for (int per_cu = 0; per_cu <= kPlanMha; per_cu++) {
-            const size_t b = plan_bytes(batch, hq, plan_splits(batch, hq, hkv, S, g, per_cu, cu), D);
-            n = b > n ? b : n;
-        }
+    auto add = [&](int g, int per_cu) {
+        const size_t b = plan_bytes(batch, hq, plan_splits(batch, hq, hkv, S, g, per_cu, cu), D);
+        n = b > n ? b : n;
+    };
+    for (int per_cu = 0; per_cu <= kPlanMha; per_cu++) add(Gmax, per_cu);
+    // (groups of eight run as two of four: the plans of their own policies only,
+    // so that the same calls fit the allocation-free entry point's scratch)
+    if (G != Gmax) {
+        add(G, kPlanFixed);
+        add(G, plan_per_cu(MODE_BINARY, D, G));
+        add(G, plan_per_cu(MODE_COMP, D, G));
+        add(G, plan_per_cu(MODE_MIXED, D, G));
+    }
     n = list_offset(n) + list_bytes((int64_t)batch * hkv * ((hq / hkv) / G));
     last = Last{batch, hq, hkv, S, D, cu, n};
     return n;

@@ -213,6 +213,28 @@ def test_workspace_covers_every_split_plan(lib):
              ctypes.byref(total)) == BC_ERR_INVALID_ARGUMENT
 
 
+def test_groups_of_eight_in_fours_take_no_more_workspace(lib):
+    """Groups of eight at d = 32, 96, 160, 192 and 224 run as two groups of
+    four: shapes whose partials fit the allocation-free entry point's 8 MiB
+    as one group fit it as two (each policy's plan of two groups is covered by
+    the size, and the split-phase plan takes as many splits as one group's)."""
+    size_t = ctypes.c_size_t
+    f = lib.bc_attention_split_plan
+    f.argtypes = [ctypes.c_int] * 7 + [ctypes.POINTER(ctypes.c_int), ctypes.POINTER(size_t),
+                                       ctypes.POINTER(size_t)]
+    n, part, total = ctypes.c_int(0), size_t(0), size_t(0)
+    for (B, Hq, Hkv, S, d), before in {(15, 128, 16, 2596, 224): 6944896, (21, 64, 4, 3760, 224): 7291456,
+                                       (1, 64, 8, 9001, 32): 252736, (8, 64, 8, 60000, 192): None}.items():
+        for mode in range(4):
+            assert f(mode, B, Hq, Hkv, S, d, 256, ctypes.byref(n), ctypes.byref(part),
+                     ctypes.byref(total)) == BC_OK, lib.bc_last_error()
+            assert part.value <= total.value
+            if before is not None:
+                # (the list of per-head modes' groups is twice as long: 8 bytes a group)
+                assert total.value <= before + 8 * B * Hq // 4 + 256, (B, Hq, Hkv, S, d)
+                assert total.value <= 8 << 20
+
+
 def test_wide_binary_plan(lib):
     """Binary MHA attention at d = 64, 128, 256 with one head per CU (and a
     context of at most 131072 keys) plans one split per head: one wide
