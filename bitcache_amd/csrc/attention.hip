@@ -1243,10 +1243,10 @@ int run_partial(int mode, const void* q, const void* k_bin, const void* k_res, c
         a.app_slot = app->slot;
     }
     const dim3 grid(p.n_splits, batch * n_kv_heads * ((n_heads / n_kv_heads) / p.G));
-    // the matrix-core kernel, but for splits past its offsets' range (the VALU
-    // kernel, selectable with BITCACHE_VALU_ATTENTION=1).  With one split per
-    // group the matrix-core kernel normalises and writes the output itself (no
-    // merge launch).
+    // the matrix-core kernel, but for splits past its offsets' range and more
+    // head groups than its plan argument holds (the VALU kernel, selectable with
+    // BITCACHE_VALU_ATTENTION=1).  With one split per group the matrix-core
+    // kernel normalises and writes the output itself (no merge launch).
     if (direct_out != nullptr && p.n_splits == 1) a.out = (uint16_t*)direct_out;
     // Per-head modes: the groups whose heads are all binary go to the binary
     // kernel, which reads none of their residual bytes, the others to the
@@ -1269,7 +1269,8 @@ int run_partial(int mode, const void* q, const void* k_bin, const void* k_res, c
         a.group_list = lists + kListHeader / sizeof(int32_t);
         a.group_count = lists;
     }
-    const bool mfma = !valu_forced() && bc::mfma_split_ok(head_dim, a.chunk);
+    const int64_t head_groups = (n_heads / n_kv_heads) / p.G;
+    const bool mfma = !valu_forced() && bc::mfma_split_ok(head_dim, a.chunk, head_groups);
     // one wide workgroup per head (wide_plan): no partials, no merge launch
     if (mfma && direct_out != nullptr && app == nullptr &&
         wide_plan(mode, head_dim, p.G, groups, seq_len, bc::device_cu_count())) {
@@ -1277,7 +1278,7 @@ int run_partial(int mode, const void* q, const void* k_bin, const void* k_res, c
         w.n_splits = 1;
         w.chunk = (seq_len + 63) / 64 * 64;
         w.out = (uint16_t*)direct_out;
-        if (bc::mfma_split_ok(head_dim, w.chunk) &&
+        if (bc::mfma_split_ok(head_dim, w.chunk, head_groups) &&
             bc::launch_mfma_split(mode, head_dim, 1, w, dim3(1, (unsigned)groups), st, kWideWaves)) {
             if (wrote_out) *wrote_out = true;
             return bc::check_launch("attention (wide workgroups)");
@@ -1528,7 +1529,7 @@ extern "C" int bc_append_attention(const void* q, const void* k_new, const void*
     const SplitPlan p = plan_splits(batch, n_heads, n_kv_heads, seq_len, G, plan_per_cu(mode, head_dim, G));
     hipStream_t st = (hipStream_t)stream;
     if (valu_forced() || G != group || !bc::append_dim(head_dim) ||
-        !bc::mfma_split_ok(head_dim, p.chunk)) {
+        !bc::mfma_split_ok(head_dim, p.chunk, 1)) {
         const int rc = bc_online_encode_kv(k_new, v_new, k_bin, k_res, v_bin, v_res, batch,
                                            n_kv_heads, head_dim, current_len, max_seq, stream);
         if (rc != BC_OK) return rc;

@@ -36,8 +36,8 @@ int mfma_wgs_per_cu(int mode, int D, int G) {
     return n;
 }
 
-bool mfma_split_ok(int D, int64_t chunk) {
-    if (!head_dim_ok(D)) return false;
+bool mfma_split_ok(int D, int64_t chunk, int64_t head_groups) {
+    if (!head_dim_ok(D) || head_groups > kMaxHeadGroups) return false;
     // buffer offsets are 32-bit and relative to a split's key range; the
     // prefetches reach up to 17 tiles (1088 keys) past its end.  The int8
     // value path adds at most 2^16 per tile to an int32 accumulator: a wave
@@ -46,7 +46,7 @@ bool mfma_split_ok(int D, int64_t chunk) {
 }
 
 bool launch_mfma_split(int mode, int D, int G, const AttnArgs& a, dim3 grid, hipStream_t st, int nw) {
-    if (!mfma_split_ok(D, a.chunk)) return false;
+    if (!mfma_split_ok(D, a.chunk, (a.Hq / a.Hkv) / G)) return false;
     // adaptive mode reads the popcounts stored by the selection passes
     if (mode == MODE_ADAPTIVE && a.pcs == nullptr) return false;
     switch (D) {

@@ -71,8 +71,11 @@ template <int D>
 bool mfma_launch(int mode, int G, const AttnArgs& a, dim3 grid, hipStream_t st, int nw);
 template <int D>
 int mfma_occupancy(int mode, int G);
-// True if the MFMA kernels handle head_dim D with splits of `chunk` keys.
-bool mfma_split_ok(int D, int64_t chunk);
+// Query-head groups per kv head that the MFMA kernels' packed plan argument holds.
+constexpr int kMaxHeadGroups = (1 << 13) - 1;
+// True if the MFMA kernels handle head_dim D with splits of `chunk` keys and
+// `head_groups` query-head groups per kv head.
+bool mfma_split_ok(int D, int64_t chunk, int64_t head_groups);
 // Head dims whose kernels append a token in place (the one-slice row encoder
 // of encode_row.h takes power-of-two lane groups).
 __host__ __device__ constexpr bool append_dim(int D) { return D == 64 || D == 128 || D == 256; }

@@ -472,7 +472,8 @@ __host__ __device__ constexpr bool k_on_mfma(int G, int mode) {
 // (bits 0..16), whether the launch's groups come from a list (bit 17) and the
 // head groups per kv head (bits 18..30).  Measured with it: one 64-key call
 // 0.9 us less.
-constexpr int kPlanList = 1 << 17, kPlanGroups = 18, kMaxHeadGroups = (1 << 13) - 1;
+constexpr int kPlanList = 1 << 17, kPlanGroups = 18;
+static_assert(((int64_t)bc::kMaxHeadGroups << kPlanGroups | (kPlanList - 1)) < ((int64_t)1 << 31), "the packed plan holds every count");
 inline int pack_plan(const AttnArgs& a, int G) {
     return a.chunk / 64 | (a.group_list != nullptr ? kPlanList : 0) | (((a.Hq / a.Hkv) / G) << kPlanGroups);
 }
@@ -1948,7 +1949,6 @@ namespace bc {
 
 template <int D>
 bool mfma_launch(int mode, int G, const AttnArgs& a, dim3 grid, hipStream_t st, int nw) {
-    if ((a.Hq / a.Hkv) / G > kMaxHeadGroups) return false;
     if (a.app_k != nullptr && (!append_dim(D) || mode == MODE_ADAPTIVE || mode == MODE_MIXED)) return false;
     if (nw != 4) return launch_wide<D>(mode, G, a, grid, st, nw);
     switch (G) {
