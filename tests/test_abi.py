@@ -266,6 +266,16 @@ def test_wide_binary_plan(lib):
     assert splits(3, 8, 32, 32, 32768, 128, 256) > 1         # per-head modes
 
 
+def test_query_preparation_is_inlined():
+    """No attention kernel calls its query preparation: a called function
+    waits for the first tile's loads, which it is meant to run beside."""
+    if not os.path.exists(LIB):
+        pytest.skip("library not built")
+    code = open(LIB, "rb").read()
+    assert b"attn_mfma_kernel" in code
+    assert not re.findall(rb"_ZN12_GLOBAL__N_111prep_digits\w*", code)
+
+
 def test_extension_rejects_cpu_tensors():
     torch = pytest.importorskip("torch")
     import bitcache_amd
