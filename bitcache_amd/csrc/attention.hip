@@ -937,10 +937,21 @@ struct SplitPlan {
 // per_cu = kPlanMha: as 0, but the launches too small for two rounds of eight
 // fill one of two workgroups per CU (4x16 heads of 9300 keys 24.5 -> 23.3 us,
 // 2x32 heads of 9973 keys, d = 96, 22.5 -> 21.2).
+//
+// per_cu = kPlanEight + n: binary groups of eight, n workgroups of which fit a CU.
+// Their fixed work (eight queries prepared, eight heads' sums merged) is that of
+// 20 to 30 tiles, and partials of eight heads make the merge launch longer than
+// another's, so a second split pays late: the model of rounds above took
+// 768x(8 heads) of 2500 keys, d = 128, in four splits (65 us; one split: 33) and
+// 512x(8 heads) of 1200 keys in two (28; 18).  The cost is us of the busiest CU
+// with w workgroups of `per` tiles, n at a time, 2 w + per (0.24 ceil(w / n) +
+// 0.08 w), and 3 + 1.2 w for the merge.  Over 8 to 1536 groups of 600 to 50000 keys its choice is within 1%
+// (d = 64), 0.3% (128, 256) of the fastest measured split in the mean.
 // `cu` is the device's CU count (0: the current device's).
 constexpr int kMaxPerCu = 4;
 constexpr int kPlanMha = kMaxPerCu + 1;
 constexpr int kShortTiles = 4;   // per wave
+constexpr int kPlanEight = 8;
 SplitPlan plan_splits(int batch, int hq, int hkv, int S, int G, int per_cu, int cu = 0) {
     SplitPlan p;
     p.G = G;
@@ -959,7 +970,25 @@ SplitPlan plan_splits(int batch, int hq, int hkv, int S, int G, int per_cu, int 
         if (alone > max_split) max_split = alone < kMaxSplits ? (int)alone : kMaxSplits;
     }
     int want = 1;
-    if (groups > 0 && tiles > 0 && per_cu > 0 && per_cu <= kMaxPerCu) {
+    if (groups > 0 && tiles > 0 && per_cu > kPlanEight) {
+        const int fit = per_cu - kPlanEight;
+        // (no more splits than two plans that ws_bytes covers)
+        const int n0 = plan_splits(batch, hq, hkv, S, G, 0, cu).n_splits;
+        const int n1 = plan_splits(batch, hq, hkv, S, G, fit, cu).n_splits;
+        const int most = n0 > n1 ? n0 : n1;
+        double best = 0.0;
+        for (int sp = 1; sp <= most; sp++) {
+            const int per = (tiles + sp - 1) / sp;
+            if ((tiles + per - 1) / per != sp) continue;   // (the same plan as a smaller count)
+            const int64_t w = (groups * sp + cu - 1) / cu;
+            const double t = 2.0 * w + per * (0.24 * ((w + fit - 1) / fit) + 0.08 * w) +
+                             (sp > 1 ? 3.0 + 1.2 * w : 0.0);
+            if (sp == 1 || t < best) {
+                best = t;
+                want = sp;
+            }
+        }
+    } else if (groups > 0 && tiles > 0 && per_cu > 0 && per_cu <= kMaxPerCu) {
         const int64_t slots = (int64_t)per_cu * cu;
         // beyond 4 rounds' worth of splits nothing improves
         const int64_t lim = 4 * slots / groups + 1;
@@ -970,7 +999,10 @@ SplitPlan plan_splits(int batch, int hq, int hkv, int S, int G, int per_cu, int 
             const int n = (tiles + per - 1) / per;
             if (n != sp) continue;               // (the same plan as a smaller count)
             const int64_t rounds = (groups * n + slots - 1) / slots;
-            const double t = (double)rounds * (per + 2);
+            // (four workgroups fit a CU: the merge launch counts, or three of one
+            // split each end up in four rounds; compensated 768x2 heads of 2500
+            // keys, d = 64, 34.1 us with one split, 36.3 with four)
+            const double t = (double)rounds * (per + 2) + (per_cu == 4 && n > 1 ? 6 : 0);
             if (sp == 1 || t < best * 0.999) {
                 best = t;
                 want = sp;
@@ -1029,17 +1061,16 @@ SplitPlan plan_splits(int batch, int hq, int hkv, int S, int G, int per_cu, int 
 // at most two (its tiles are short, so a workgroup's fixed prologue and
 // epilogue weigh more than the latency hiding of a third: c2 54.5 -> 52.9 us).
 //
-// kPlanMha bounds every policy: ws_bytes sizes the workspace over the plans
-// of per_cu = 0 .. kPlanMha, so a policy above it would launch more splits
-// than the workspace holds.
+// ws_bytes sizes the workspace over the plans of per_cu = 0 .. kPlanMha; the
+// policy of binary groups of eight never takes more splits than those.
 int plan_per_cu(int mode, int D, int G) {
     if ((mode == MODE_COMP || mode == MODE_MIXED) && G == 1) return kPlanMha;
     // (MHA binary 2, GQA binary 4, the other modes 3, and 4 up to d = 64,
     // where four workgroups fit: 8x(32/8) heads of 20011 keys 26.8 -> 25.7 us)
     int cap = mode == MODE_BINARY ? (G == 1 ? 2 : 4) : (D <= 64 ? 4 : 3);
-    if (cap > kMaxPerCu) cap = kMaxPerCu;
     const int n = bc::mfma_wgs_per_cu(mode, D, G);
-    return n <= 0 ? cap : (n < cap ? n : cap);
+    if (n > 0 && n < cap) cap = n;
+    return mode == MODE_BINARY && G == 8 ? kPlanEight + cap : cap;
 }
 // the policy of the split-phase entry points (bc_attention_partial and
 // bc_attention_combine, which does not know the mode), and of the fp16

@@ -266,6 +266,33 @@ def test_wide_binary_plan(lib):
     assert splits(3, 8, 32, 32, 32768, 128, 256) > 1         # per-head modes
 
 
+def test_one_split_where_the_merge_costs_more(lib):
+    """Launches of at least one and a half workgroups per CU over short
+    contexts keep one split per group (no partials, no merge launch): binary
+    groups of eight, and compensated groups of two at d = 64."""
+    n, part, ws = ctypes.c_int(), ctypes.c_size_t(), ctypes.c_size_t()
+
+    def splits(mode, b, h, hk, s, d):
+        assert lib.bc_attention_split_plan(mode, b, h, hk, s, d, 256, ctypes.byref(n),
+                                           ctypes.byref(part), ctypes.byref(ws)) == BC_OK
+        assert part.value <= ws.value
+        return n.value
+
+    for d in (64, 128, 256):
+        for batch, seq in ((48, 2500), (64, 1200), (96, 2500), (96, 5000), (128, 5000), (192, 1200)):
+            assert splits(0, batch, 64, 8, seq, d) == 1
+        assert splits(0, 1, 64, 8, 50000, d) >= 16          # a CU for every workgroup
+        assert 4 <= splits(0, 8, 64, 8, 9001, d) <= 12
+        assert splits(0, 64, 64, 8, 18000, d) > 1
+    assert splits(1, 96, 16, 8, 2500, 64) == 1
+    assert splits(1, 192, 16, 8, 1200, 64) == 1
+    for mode in (0, 1, 2, 3):                                # and the workspace holds every plan
+        for d in (64, 128, 256):
+            for batch in (1, 3, 8, 17, 50, 96, 97, 200):
+                for seq in (1, 64, 700, 4097, 33333, 131072, 1000000):
+                    splits(mode, batch, 64, 8, seq, d)
+
+
 def test_query_preparation_is_inlined():
     """No attention kernel calls its query preparation: a called function
     waits for the first tile's loads, which it is meant to run beside."""
