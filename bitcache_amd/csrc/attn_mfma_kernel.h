@@ -403,8 +403,8 @@ __device__ __forceinline__ void prep_digits(const uint16_t (&qpre)[NQ], QDigits<
 // Build-time switches; each default is the measured fastest on MI355X:
 //   BC_MHA_WAVES   waves/SIMD the MHA compensated kernel's registers target (3)
 //   BC_BIN_WAVES   the same for binary attention of groups up to 2 (5)
-//   BC_ADAPT_WAVES the same for adaptive attention up to d = 128 (2; its LDS
-//                  holds two workgroups per CU at d = 128)
+//   BC_ADAPT_WAVES the same for adaptive attention (2 where Occupancy::kAdaptTwo;
+//                  its LDS holds two workgroups per CU at d = 128)
 //   BC_LIN_V       V code tiles read as linear KiB runs (1) instead of per key
 //   BC_MHA_PIPE / BC_ADAPT_PIPE / BC_GQA_PIPE  one-tile prefetch with two staging
 //                  buffers for MHA (1), adaptive (1) and GQA compensated (0: one
@@ -448,9 +448,14 @@ struct Occupancy {
     // groups of 2 29 / 34; d = 224 groups of 4 36.5 / 40.6), one where they
     // do not (d = 256, groups of 4: 37.4 us at one, 47.0 at two)
     static constexpr bool kTwo = G <= 2 || (G == 4 && D <= 224) || D <= 160;
+    // Adaptive heads: two up to d = 128 and for single heads of d = 160, whose
+    // operands fit 256 registers (2048 heads of 800 keys 174 us at one, 121 at
+    // two; 128 heads of 8000 keys 72 / 59); spilling costs the others what two
+    // bring (d = 192 MHA, 2048 heads of 600 keys 177 / 145, 256 of 800 42 / 46)
+    static constexpr bool kAdaptTwo = D <= 128 || (D == 160 && G == 1);
     static constexpr int kWaves =
         MODE == MODE_BINARY     ? (D <= 128 ? (G <= 2 ? BC_BIN_WAVES : 3) : 2)
-        : MODE == MODE_ADAPTIVE ? (D <= 128 ? BC_ADAPT_WAVES : 1)
+        : MODE == MODE_ADAPTIVE ? (kAdaptTwo ? BC_ADAPT_WAVES : 1)
         : (G == 1 && D <= 128)  ? BC_MHA_WAVES
                                 : (D <= 128 ? (G <= 4 && !BC_GQA_PIPE ? 3 : 2) : (kTwo ? 2 : 1));
 };
