@@ -1001,7 +1001,7 @@ SplitPlan plan_splits(int batch, int hq, int hkv, int S, int G, int per_cu, int 
             const int64_t rounds = (groups * n + slots - 1) / slots;
             // (four workgroups fit a CU: the merge launch counts, or three of one
             // split each end up in four rounds; compensated 768x2 heads of 2500
-            // keys, d = 64, 34.1 us with one split, 36.3 with four)
+            // keys, d = 64, 28.8 us with one split, 36.4 with four)
             const double t = (double)rounds * (per + 2) + (per_cu == 4 && n > 1 ? 6 : 0);
             if (sp == 1 || t < best * 0.999) {
                 best = t;
@@ -1110,6 +1110,30 @@ bool valu_forced() {
         return e != nullptr && e[0] == '1';
     }();
     return forced;
+}
+
+// Contexts up to which the VALU kernel runs instead of the matrix-core one, in
+// keys per group and CU: many single heads (or pairs) of d >= 160 over little
+// more than a tile.  A matrix-core workgroup's cost is then that of its query
+// preparation, a whole tile for any key of it and its epilogue at one or two
+// waves per SIMD; the VALU kernel's grows with the keys and has more in flight.
+// us, VALU / matrix cores, 256 CUs:
+//   adaptive single heads d = 224  512 of 128 keys 43.2 / 45.9, of 400 56.9 / 53.5;
+//                         2048 of 17 keys 84 / 135, of 400 162 / 173, of 600 200.5 / 199.5
+//                         d = 192  512 of 128 40.8 / 43.0; 2048 of 17 73.5 / 120, of 600 157 / 177
+//                         d = 160  2048 of 17 71.7 / 81.4, of 64 81.5 / 82.2, 512 of 17 35.7 / 32.4
+//            pairs        d = 192  512 of 17 46.9 / 49.8, of 64 47.7 / 49.4; 2048 of 200 163 / 168
+//   compensated single heads       2048 of 17 24.3 / 28.6, 25.4 / 30.0, 27.6 / 36.0 (d = 160, 192,
+//                         224), of 40 27.8 / 28.9, 29.9 / 30.2, 34.7 / 36.2, of 64 33.6 / 28.9,
+//                         37.6 / 30.6, 42.0 / 36.1; 512 of 17 12.6 / 9.2
+int valu_keys_per_group(int mode, int D, int G) {
+    if (mode == MODE_ADAPTIVE && G == 1) return D == 192 || D == 224 ? 72 : (D == 160 ? 8 : 0);
+    if (mode == MODE_ADAPTIVE && G == 2) return D == 192 ? 32 : 0;
+    if (mode == MODE_COMP && G == 1) return D == 160 || D == 192 || D == 224 ? 5 : 0;
+    return 0;
+}
+bool valu_better(int mode, int D, int G, int64_t groups, int S, int cu) {
+    return groups >= 2LL * cu && (int64_t)S * cu <= valu_keys_per_group(mode, D, G) * groups;
 }
 
 // bytes of the split partials a plan writes: one (max, sum, acc[D]) fp32
@@ -1274,9 +1298,9 @@ int run_partial(int mode, const void* q, const void* k_bin, const void* k_res, c
         a.app_slot = app->slot;
     }
     const dim3 grid(p.n_splits, batch * n_kv_heads * ((n_heads / n_kv_heads) / p.G));
-    // the matrix-core kernel, but for splits past its offsets' range and more
-    // head groups than its plan argument holds (the VALU kernel, selectable with
-    // BITCACHE_VALU_ATTENTION=1).  With one split per group the matrix-core
+    // the matrix-core kernel, but for short contexts of many heads (valu_better),
+    // splits past its offsets' range and more head groups than its plan argument
+    // holds (the VALU kernel, selectable with BITCACHE_VALU_ATTENTION=1).  With one split per group the matrix-core
     // kernel normalises and writes the output itself (no merge launch).
     if (direct_out != nullptr && p.n_splits == 1) a.out = (uint16_t*)direct_out;
     // Per-head modes: the groups whose heads are all binary go to the binary
@@ -1301,7 +1325,9 @@ int run_partial(int mode, const void* q, const void* k_bin, const void* k_res, c
         a.group_count = lists;
     }
     const int64_t head_groups = (n_heads / n_kv_heads) / p.G;
-    const bool mfma = !valu_forced() && bc::mfma_split_ok(head_dim, a.chunk, head_groups);
+    const bool mfma = !valu_forced() &&
+                      !valu_better(mode, head_dim, p.G, groups, seq_len, bc::device_cu_count()) &&
+                      bc::mfma_split_ok(head_dim, a.chunk, head_groups);
     // one wide workgroup per head (wide_plan): no partials, no merge launch
     if (mfma && direct_out != nullptr && app == nullptr &&
         wide_plan(mode, head_dim, p.G, groups, seq_len, bc::device_cu_count())) {
