@@ -45,8 +45,7 @@ CASES = [
     # passes over key chunks of 1024 (several per head), without and with ties
     (16, 32, 8, 8192, 128, 820, False),
     (16, 32, 8, 8192, 128, 820, True),
-    # head dims without the matrix-core kernel (the VALU split kernel's
-    # adaptive mode), MHA and GQA
+    # head dims other than 64, 128 and 256, MHA and GQA
     (1, 2, 2, 300, 32, 30, False),
     (1, 8, 2, 520, 32, 52, True),
     (1, 4, 4, 900, 96, 90, False),

@@ -562,7 +562,7 @@ def test_gqa_equals_mha_on_repeated_kv(F, group, d):
                                           # more query-head groups than one block of the
                                           # group compaction takes at a time (1024)
                                           (40, 32, 32, 130, 64), (48, 32, 8, 200, 128),
-                                          # the VALU kernel's per-head modes
+                                          # head dims other than 64, 128 and 256
                                           (1, 4, 4, 500, 32), (1, 8, 2, 600, 96),
                                           (1, 4, 2, 300, 160), (1, 8, 4, 250, 224)])
 def test_head_mode_attention(F, B, Hq, Hkv, S, d):

@@ -12,8 +12,8 @@ nats, in which case it also adds the low 8 bits.  The rounding error per
 element is then at most step/2, the same absolute bound on every element, so
 elements far below max|q| keep fewer significant bits; these cases bound what
 that costs on the outputs: compensated MHA and GQA, adaptive top-k (whose
-selection uses only the exact binary key) and per-head modes, at d = 64, 128
-and 256, plus the VALU kernel's head dims (fp32 residual dot)."""
+selection uses only the exact binary key) and per-head modes, at d = 64, 96,
+128, 160 and 256."""
 import numpy as np
 import pytest
 import torch
@@ -73,7 +73,7 @@ SHAPES = [
     (1, 8, 4, 600, 128),    # GQA 2
     (1, 16, 2, 300, 128),   # GQA 8
     (1, 8, 2, 400, 256),    # GQA 4
-    (1, 4, 4, 300, 96),     # VALU kernel (fp32 residual dot)
+    (1, 4, 4, 300, 96),     # rows of no power of two of code pieces
     (1, 8, 2, 260, 160),
 ]
 
@@ -104,7 +104,7 @@ def test_compensated_and_adaptive_with_extreme_queries(shape, kind):
     for (b, h), idx in sets.items():
         assert np.array_equal(np.nonzero(sel[b, h])[0], idx), f"set differs at ({b}, {h})"
     close(to_np(aout).astype(np.float32), aref, what=f"adaptive {kind} {shape}")
-    # per-head modes (the matrix-core kernel at 64/128/256, the VALU one otherwise)
+    # per-head modes
     modes = torch.from_numpy((np.arange(B * Hq) % 2).astype(np.uint8).reshape(B, Hq)).cuda()
     mout = F.head_mode_attention(qt, kb, kr, vb, vr, modes, B, Hq, S, d, n_kv_heads=Hkv)
     _, bref = O.binary_attention(q, Kb, Vb, B, Hq, S, n_kv_heads=Hkv, return_f32=True)

@@ -78,7 +78,7 @@ def _tok(rng, shape, sigma=0.3):
     (1, 1, 128, 64, 40, True),      # B*H = 1, partly filled
     (1, 1, 64, 32, 9, False),       # B*H = 1, partly filled, binary mode (aliased residual)
     (2, 4, 128, 64, 40, True),      # B*H > 1, partly filled
-    (2, 3, 96, 48, 17, True),       # B*H > 1, head dim without the matrix-core kernel
+    (2, 3, 96, 48, 17, True),       # B*H > 1, a head dim other than 64, 128, 256
     (1, 4, 256, 40, 23, False),     # B*H > 1, binary mode
     (2, 4, 64, 16, 37, True),       # full ring, wrapped twice
     (1, 2, 128, 32, 70, False),     # full ring, binary mode
