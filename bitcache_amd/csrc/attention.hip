@@ -1056,10 +1056,12 @@ SplitPlan plan_splits(int batch, int hq, int hkv, int S, int G, int per_cu, int 
 
 // The split policy of a full attention call (plan_splits' per_cu): MHA
 // compensated attention several rounds; binary, GQA compensated and adaptive
-// attention one round of what fits of their kernel, at most three workgroups
-// per CU (the adaptive kernel's LDS allows two at d = 128), binary attention
-// at most two (its tiles are short, so a workgroup's fixed prologue and
-// epilogue weigh more than the latency hiding of a third: c2 54.5 -> 52.9 us).
+// attention one round of what fits of their kernel: at most three workgroups
+// per CU (the adaptive kernel's LDS allows two at d = 128), four up to d = 64
+// and in binary groups of 2 and 4, two in MHA binary attention (its tiles are
+// short, so a workgroup's fixed prologue and epilogue weigh more than the
+// latency hiding of a third: c2 54.5 -> 52.9 us), and kPlanEight for binary
+// groups of eight.
 //
 // ws_bytes sizes the workspace over the plans of per_cu = 0 .. kPlanMha; the
 // policy of binary groups of eight never takes more splits than those.
@@ -1112,28 +1114,29 @@ bool valu_forced() {
     return forced;
 }
 
-// Contexts up to which the VALU kernel runs instead of the matrix-core one, in
-// keys per group and CU: many single heads (or pairs) of d >= 160 over little
-// more than a tile.  A matrix-core workgroup's cost is then that of its query
-// preparation, a whole tile for any key of it and its epilogue at one or two
-// waves per SIMD; the VALU kernel's grows with the keys and has more in flight.
-// us, VALU / matrix cores, 256 CUs:
-//   adaptive single heads d = 224  512 of 128 keys 43.2 / 45.9, of 400 56.9 / 53.5;
+// Where the VALU kernel runs instead of the matrix-core one: many single heads
+// (or pairs) over contexts of little more than a tile, up to `base` keys and
+// `per` more for each group per CU.  A matrix-core workgroup's cost is then that
+// of its query preparation, a whole tile for any key of it and its epilogue, at
+// one or two waves per SIMD above d = 128; the VALU kernel's grows with the keys
+// and has more in flight.  us, VALU / matrix cores, 256 CUs:
+//   adaptive single heads d = 224  512 of 260 keys 48.9 / 52.0, of 400 56.9 / 53.5;
 //                         2048 of 17 keys 84 / 135, of 400 162 / 173, of 600 200.5 / 199.5
-//                         d = 192  512 of 128 40.8 / 43.0; 2048 of 17 73.5 / 120, of 600 157 / 177
+//                         d = 192  512 of 260 45.0 / 48.2, of 400 52.8 / 49.3;
+//                         2048 of 17 73.5 / 120, of 600 157 / 177
 //                         d = 160  2048 of 17 71.7 / 81.4, of 64 81.5 / 82.2, 512 of 17 35.7 / 32.4
-//            pairs        d = 192  512 of 17 46.9 / 49.8, of 64 47.7 / 49.4; 2048 of 200 163 / 168
+//                         d = 96   2048 of 17 62.3 / 71.2, of 64 67.3 / 72.0, of 130 75.2 / 76.0
+//            pairs        d = 192  512 of 17 46.9 / 49.8, of 64 47.7 / 49.4; 2048 of 260 179 / 183
 //   compensated single heads       2048 of 17 24.3 / 28.6, 25.4 / 30.0, 27.6 / 36.0 (d = 160, 192,
 //                         224), of 40 27.8 / 28.9, 29.9 / 30.2, 34.7 / 36.2, of 64 33.6 / 28.9,
 //                         37.6 / 30.6, 42.0 / 36.1; 512 of 17 12.6 / 9.2
-int valu_keys_per_group(int mode, int D, int G) {
-    if (mode == MODE_ADAPTIVE && G == 1) return D == 192 || D == 224 ? 72 : (D == 160 ? 8 : 0);
-    if (mode == MODE_ADAPTIVE && G == 2) return D == 192 ? 32 : 0;
-    if (mode == MODE_COMP && G == 1) return D == 160 || D == 192 || D == 224 ? 5 : 0;
-    return 0;
-}
 bool valu_better(int mode, int D, int G, int64_t groups, int S, int cu) {
-    return groups >= 2LL * cu && (int64_t)S * cu <= valu_keys_per_group(mode, D, G) * groups;
+    int per = 0, base = 0;
+    if (mode == MODE_ADAPTIVE && G == 1 && (D == 192 || D == 224)) per = 56, base = 176;
+    if (mode == MODE_ADAPTIVE && G == 1 && (D == 96 || D == 160)) per = 8;
+    if (mode == MODE_ADAPTIVE && G == 2 && D == 192) per = 32;
+    if (mode == MODE_COMP && G == 1 && (D == 160 || D == 192 || D == 224)) per = 5;
+    return per > 0 && groups >= 2LL * cu && (int64_t)(S - base) * cu <= per * groups;
 }
 
 // bytes of the split partials a plan writes: one (max, sum, acc[D]) fp32

@@ -1,4 +1,4 @@
-"""Many heads of d >= 160 over short contexts: calls just inside and just past
+"""Many single heads and pairs over short contexts: calls just inside and just past
 the contexts that run on the VALU split kernel, against the oracle."""
 import numpy as np
 import pytest
@@ -10,8 +10,9 @@ from tests.gpu_util import bin_from_blob, close, res_from_blob, say, to_np
 pytestmark = pytest.mark.gpu
 
 # (mode, d, group, kv heads of one sequence, contexts around the line on 256 CUs)
-CASES = [("adaptive", 192, 1, 512, (1, 17, 144, 145)), ("adaptive", 224, 1, 1024, (63, 288, 289)),
-         ("adaptive", 160, 1, 2048, (17, 64, 65)), ("adaptive", 192, 2, 512, (64, 65)),
+CASES = [("adaptive", 192, 1, 512, (1, 17, 288, 289)), ("adaptive", 224, 1, 1024, (63, 400, 401)),
+         ("adaptive", 160, 1, 2048, (17, 64, 65)), ("adaptive", 96, 1, 2048, (64, 65)),
+         ("adaptive", 192, 2, 512, (64, 65)),
          ("compensated", 160, 1, 2048, (17, 40, 41)), ("compensated", 192, 1, 2048, (40, 41)),
          ("compensated", 224, 1, 2048, (1, 40, 41))]
 
