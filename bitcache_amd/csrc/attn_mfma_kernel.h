@@ -1335,7 +1335,7 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
             // (a scale that is not finite takes no part: the heads that read it are
             // NaN whatever the plan, a head that reads only the key's other part
             // needs its weights planned all the same)
-            const float wa = 2.0f * svv, wr = rsv * (1.0f / 7.0f);
+            const float wa = 2.0f * fabsf(svv), wr = fabsf(rsv) * (1.0f / 7.0f);
             const float wb = valid ? fmaxf(wa < INFINITY ? wa : 0.0f, wr < INFINITY ? wr : 0.0f) : 0.0f;
             if (__ballot(wb > wlim) != 0ull) {
                 const float wmx = wave_max(wb);
@@ -1412,10 +1412,10 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
             if constexpr (I8) {
                 ps[g] = p * es[g];
                 wsig[g] = fmaf(ps[g], fa, 0.5f);
-                wtop = fmaxf(wtop, wsig[g]);
+                wtop = fmaxf(wtop, fabsf(wsig[g]));
                 if constexpr (RES) {
                     wresid[g] = fmaf(ps[g], with_res(g) ? fb : 0.0f, 0.5f);
-                    wtop = fmaxf(wtop, wresid[g]);
+                    wtop = fmaxf(wtop, fabsf(wresid[g]));
                 }
             } else {
                 const float a2 = p * fa;
@@ -1443,8 +1443,8 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
                 uint32_t wmx[G];
 #pragma unroll
                 for (int g = 0; g < G; g++) {
-                    float w = wsig[g] < INFINITY ? wsig[g] : 0.0f;
-                    if constexpr (RES) w = fmaxf(w, wresid[g] < INFINITY ? wresid[g] : 0.0f);
+                    float w = fabsf(wsig[g]) < INFINITY ? fabsf(wsig[g]) : 0.0f;
+                    if constexpr (RES) w = fmaxf(w, fabsf(wresid[g]) < INFINITY ? fabsf(wresid[g]) : 0.0f);
                     wmx[g] = __builtin_bit_cast(uint32_t, w);
                 }
                 wave_umax(wmx);
@@ -1469,21 +1469,22 @@ void attn_mfma_kernel(const uint16_t* q, const uint8_t* k_signs, const uint8_t* 
             // a V scale that is not finite has no integer weight: it makes the
             // offset, so the output of the heads that read it, NaN, as the sums
             // of the fp16 path are
-            if (__ballot(!(svv + (RES ? rsv : 0.0f) < INFINITY)) != 0ull) {
+            if (__ballot(!(fabsf(svv) + (RES ? fabsf(rsv) : 0.0f) < INFINITY)) != 0ull) {
 #pragma unroll
                 for (int g = 0; g < G; g++) off[g] += svv * 0.0f + (with_res(g) ? rsv * 0.0f : 0.0f);
             }
 #pragma unroll
             for (int g = 0; g < G; g++) {
-                // (weights are not negative: truncation after adding 1/2 rounds)
-                const uint32_t w = (uint32_t)(int)wsig[g];
+                // (truncation after adding 1/2 rounds; a scale that is negative, as no
+                // encoder writes one, rounds up)
+                const int w = (int)wsig[g];
                 // the offset a = a2 / 2 of each key, taken off at the end: half the
                 // rounded weight, so that the key's sum stays +-a of one a (half
                 // the unrounded one moves every dimension of the head the same
                 // way, by the rounding errors of all keys)
                 off[g] = fmaf(0.5f, (float)w, off[g]);
                 // balanced digits
-                dsig[g] = (w + 0x80808080u) ^ 0x80808080u;
+                dsig[g] = ((uint32_t)w + 0x80808080u) ^ 0x80808080u;
                 if constexpr (RES) dres[g] = ((uint32_t)(int)wresid[g] + 0x80808080u) ^ 0x80808080u;
             }
         }

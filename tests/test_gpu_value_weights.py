@@ -170,6 +170,30 @@ def test_residual_scale_not_finite(G):
 
 
 @pytest.mark.parametrize("mode", ["binary", "compensated", "adaptive", "mixed"])
+@pytest.mark.parametrize("G", [1, 2, 4, 8])
+def test_negative_value_scales(mode, G):
+    """V scales of either sign, which no encoder writes and a blob may hold:
+    the values are the scales' products with the signs and codes as ever."""
+    from bitcache_amd import layout
+    B, Hkv, S, d = 1, 2, 3000, 128
+    Hq = Hkv * G
+    for share in (1, 3):   # every scale negative, every third one
+        say(f"case negative V scales {mode} group {G}, one in {share}")
+        q, blobs, enc = make(B, Hq, Hkv, S, d, 4.0, 1, seed=G)
+        for kv in range(Hkv):
+            for planes, blob in ((layout.binary_planes, blobs[2]), (layout.residual_planes, blobs[3])):
+                planes(blob, d)[1][kv * S:(kv + 1) * S][::share] *= -1
+        flip = torch.ones((S, 1), dtype=torch.float64, device="cuda")
+        flip[::share] = -1
+        v = (enc[1][0], enc[1][1] * flip, enc[1][2], enc[1][3] * flip)
+        out, with_res = attend(mode, q, blobs, B, Hq, Hkv, S, d)
+        want = exact(q[0, :G], enc[0], v, with_res)
+        got = out[0, :G].double()
+        err = float(((got - want).norm(dim=-1) / want.norm(dim=-1)).max())
+        assert err <= BAR, f"error {err:.2e}"
+
+
+@pytest.mark.parametrize("mode", ["binary", "compensated", "adaptive", "mixed"])
 @pytest.mark.parametrize("shape", [(1, 8, 8, 16384, 96), (1, 8, 2, 16384, 64), (2, 32, 8, 16384, 128),
                                    (1, 16, 2, 16384, 128), (1, 4, 2, 9000, 256), (8, 32, 32, 65536, 128)],
                          ids=lambda s: str(s))
